@@ -29,6 +29,15 @@ int ws_get(la_ctx *ctx, int id, size_t bytes, void **out) {
         size_t total = bytes;
         for (int i = 0; i < WS_COUNT; ++i)
             if (i != id) total += ctx->ws[i].size;
+        Workspace &opt = ctx->ws[WS_PUB];
+        if (ctx->ws_limit > 0 && (int64_t)total > ctx->ws_limit && id != WS_PUB && opt.ptr) {
+            // the optional slot makes room
+            hipError_t e = hipStreamSynchronize(ctx->stream);
+            if (e != hipSuccess) return hip_fail(ctx, e, "ws_get sync");
+            total -= opt.size;
+            (void)hipFree(opt.ptr);
+            opt = Workspace();
+        }
         if (ctx->ws_limit > 0 && (int64_t)total > ctx->ws_limit)
             return set_error(ctx, LA_ERR_NOMEM, "workspace limit exceeded");
         if (w.ptr) {
@@ -48,6 +57,15 @@ int ws_get(la_ctx *ctx, int id, size_t bytes, void **out) {
     }
     *out = w.ptr;
     return LA_OK;
+}
+
+void *ws_try(la_ctx *ctx, int id, size_t bytes) {
+    void *p = nullptr;
+    const std::string before = ctx->last_error;
+    if (ws_get(ctx, id, bytes, &p) == LA_OK) return p;
+    (void)hipGetLastError();
+    ctx->last_error = before;
+    return nullptr;
 }
 
 static hipEvent_t ev_take(la_ctx *ctx) {

@@ -20,62 +20,10 @@
 // Once the remaining rows fit the CUs reserved for panels (the panel
 // stream's), outer blocks overlap: block j+1's panels run on those CUs while
 // the other CUs apply block j (look-ahead; see getrf_core).
-#include "la_common.hpp"
+#include "lu_device.hpp"
 #include <mutex>
 
 namespace lahip {
-
-constexpr int PANEL_MAXP = 256;     // max cooperative workgroups in a panel
-constexpr int NB_IN = 64;           // inner panel width
-constexpr int NB_OUT = 256;         // outer block width (trailing GEMM K)
-
-// ---------------------------------------------------------------- keys
-// Ordered key for |v|: NaN -> 0 (never wins), otherwise bits(|v|)+1, so that
-// unsigned comparison of keys is comparison of |v| and 0 beats NaN.
-__device__ inline uint64_t abs_key(double v) {
-    if (v != v) return 0;
-    return (uint64_t)(__double_as_longlong(v) & 0x7fffffffffffffffLL) + 1;
-}
-__device__ inline uint64_t abs_key(float v) {
-    if (v != v) return 0;
-    return (uint64_t)(__float_as_uint(v) & 0x7fffffffu) + 1;
-}
-constexpr uint64_t KEY_MAX = 0x7fffffffffffffffULL;
-constexpr uint64_t TAG_BIT = 0x8000000000000000ULL;
-constexpr int IDX_NONE = 0x7fffffff;
-
-__device__ inline bool better(uint64_t k1, int i1, uint64_t k0, int i0) {
-    return k1 > k0 || (k1 == k0 && i1 < i0);
-}
-
-// Maximum of an unsigned value over the wavefront, by DPP row shifts and
-// row broadcasts (no LDS round trip): lane 63 ends with the maximum, which
-// every lane receives.
-__device__ inline uint32_t wave_max_u32(uint32_t v)
-{
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
-    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
-// Wavefront argmax under better(): largest 64-bit key, lowest index among
-// equal keys; every lane returns the winner.  Three DPP maxima (high key
-// word, low key word among the lanes at the high maximum, complemented
-// index among the lanes at the full maximum) instead of a shuffle tree.
-__device__ inline void wave_argmax(uint64_t &key, int &idx) {
-    const uint32_t hi = (uint32_t)(key >> 32), lo = (uint32_t)key;
-    const uint32_t mhi = wave_max_u32(hi);
-    const bool at_hi = hi == mhi;
-    const uint32_t mlo = wave_max_u32(at_hi ? lo : 0u);
-    const bool at_max = at_hi && lo == mlo;
-    const uint32_t nidx = wave_max_u32(at_max ? ~(uint32_t)idx : 0u);
-    key = ((uint64_t)mhi << 32) | mlo;
-    idx = (int)~nidx;
-}
 
 // Value of row r of a wave's rows (lane r % 64, register r / 64) broadcast
 // to every lane; r is the same in every lane.
@@ -119,16 +67,6 @@ __device__ inline int64_t shfl_i64(int64_t v, int src_lane) {
 
 __device__ inline double shfl_t(double v, int src_lane) { return __shfl(v, src_lane); }
 __device__ inline float shfl_t(float v, int src_lane) { return __shfl(v, src_lane); }
-
-__device__ inline uint64_t ld_relaxed(const uint64_t *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void st_relaxed(uint64_t *p, uint64_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline int ld_status(const int32_t *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // Net row movement of a panel, computed by one wave entirely in registers:
 // lane l holds entry l (panel row kglob+l) and extra entry l (a row below
@@ -670,6 +608,20 @@ void k_getrf_panel(T *A, int64_t lda, int M, int NB, int R, int kglob, int64_t *
     if (w == 0 && wave == 1) invert_unit_lower_wave<T>(blk, LDB, NB, linv);
 }
 
+// L11^-1 of the block's 64 x 64 diagonal triangles (one workgroup each), for
+// U12, from the factored block (Lblk, nbo columns).
+template <typename T>
+__global__ __launch_bounds__(256)
+void k_block_linv(const T *Lblk, int64_t lda, int nbo, T *linv)
+{
+    __shared__ T L[NB_IN * (NB_IN + 1)];
+    const int b = blockIdx.x, nb = min(NB_IN, nbo - b * NB_IN);
+    stage_block(L, NB_IN + 1, Lblk + (int64_t)b * NB_IN * (lda + 1), lda, nb, nb);
+    __syncthreads();
+    if (threadIdx.x < 64)
+        invert_unit_lower_wave<T>(L, NB_IN + 1, nb, linv + (size_t)b * NB_IN * NB_IN);
+}
+
 // ------------------------------------------------------ single-WG panel
 // Used when the whole M x NB panel fits one workgroup's LDS.  Column j is
 // formed LEFT-looking in exactly the reference's operation order
@@ -822,6 +774,55 @@ void k_apply_rowmoves(T *A, int64_t lda, int n, int c_lo, int c_hi,
             for (int e = tid >> 6; e < cnt; e += blockDim.x >> 6)
                 A[s_dst[e] * lda + col] = tile[e][cl];
     }
+}
+
+// The same for the single map of a whole outer block (k_getrf_block), at
+// most BLK_MAP_MAX rows.  Each workgroup handles one 128-byte segment of
+// every moved row; a thread loads all its values before the barrier and
+// stores them after it, so no row is overwritten before it is read and every
+// load is in flight at once.
+template <typename T>
+__global__ __launch_bounds__(256)
+void k_block_rowmoves(T *A, int64_t lda, int n, int c_lo, int c_hi, const int64_t *map,
+                      uint64_t *perm)
+{
+    constexpr int LPR = 128 / (int)sizeof(T), RPP = 256 / LPR, VPT = BLK_MAP_MAX / RPP;
+    __shared__ int s_dst[BLK_MAP_MAX], s_src[BLK_MAP_MAX];
+    const int tid = threadIdx.x;
+    const int cnt = min((int)map[0], BLK_MAP_MAX);
+    if (cnt == 0) return;
+    for (int e = tid; e < cnt; e += 256) {
+        s_dst[e] = (int)map[1 + 2 * e];
+        s_src[e] = (int)map[2 + 2 * e];
+    }
+    __syncthreads();
+    if (blockIdx.x == gridDim.x - 1 && perm) {
+        uint64_t pv[BLK_MAP_MAX / 256];
+#pragma unroll
+        for (int k = 0; k < BLK_MAP_MAX / 256; ++k) pv[k] = perm[s_src[min(tid + 256 * k, cnt - 1)]];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < BLK_MAP_MAX / 256; ++k)
+            if (tid + 256 * k < cnt) perm[s_dst[tid + 256 * k]] = pv[k];
+        return;
+    }
+    const int v = blockIdx.x * LPR + tid % LPR;
+    const bool valid = v < c_lo + (n - c_hi);
+    const int col = !valid ? 0 : v < c_lo ? v : v + (c_hi - c_lo);
+    T rv[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+        if (k * RPP < cnt) {
+            const int e = min(tid / LPR + k * RPP, cnt - 1);
+            rv[k] = A[(int64_t)s_src[e] * lda + col];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+        if (k * RPP < cnt) {
+            const int e = tid / LPR + k * RPP;
+            if (e < cnt && valid) A[(int64_t)s_dst[e] * lda + col] = rv[k];
+        }
 }
 
 // ------------------------------------------------------------ unit TRSM
@@ -1227,8 +1228,52 @@ constexpr size_t panel_ws_bytes(size_t elem)
 {
     return ws_align((size_t)2 * PANEL_MAXP * CAND_WORDS * sizeof(uint64_t)) + ws_align(256) +
            ws_align((size_t)2 * 2 * NB_IN * sizeof(uint64_t)) +
-           ws_align((size_t)(1 + 4 * NB_IN) * sizeof(int64_t)) +
+           ws_align((size_t)(1 + 2 * BLK_MAP_MAX) * sizeof(int64_t)) +
+           ws_align((size_t)NB_OUT * sizeof(uint64_t)) +
            ws_align((size_t)(NB_OUT / NB_IN) * NB_IN * NB_IN * elem);
+}
+
+// Fixed scratch of la_dgetrf_noalloc_dev: panel workspace, swap list,
+// published multipliers.
+constexpr int64_t NOALLOC_MAX_K = 65536;
+constexpr size_t NOALLOC_PANEL_BYTES = panel_ws_bytes(sizeof(double));
+constexpr size_t NOALLOC_PUB_OFF = NOALLOC_PANEL_BYTES + NOALLOC_MAX_K * sizeof(int64_t);
+constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PUB_OFF + BLK_PUB_BYTES;
+
+// The block (M rows, nbo columns at Ablk) in one launch, then its L11^-1
+// blocks.  One workgroup per CU at most (the tall layouts fill a CU's
+// registers), nbo / cw of them, all resident at once on the whole device or
+// on the panel stream's CUs (checked by the caller).
+template <typename T>
+static int launch_block(la_ctx *ctx, const BlockCfg &cfg, T *Ablk, int64_t lda, int M, int nbo,
+                        int kglob, int64_t *d_ipiv, T *pub, uint64_t *pv, int64_t *map,
+                        int32_t *d_status, uint64_t ticks, T *linvs)
+{
+    {
+        ProfScope ps(ctx, LA_K_PANEL, (double)M * nbo * nbo, 2.0 * M * nbo * sizeof(T));
+        void *args[] = {&Ablk, &lda, &M, &nbo, &kglob, &d_ipiv, &pub, &pv, &map, &d_status, &ticks};
+        LA_HIP_CHECK(ctx, hipLaunchKernel(cfg.fn, dim3((unsigned)ceil_div(nbo, cfg.cw)),
+                                          dim3(cfg.nt), args, cfg.lds, ctx->stream));
+    }
+    hipLaunchKernelGGL(k_block_linv<T>, dim3((unsigned)ceil_div(nbo, NB_IN)), dim3(256), 0,
+                       ctx->stream, (const T *)Ablk, lda, nbo, linvs);
+    LA_HIP_CHECK(ctx, hipGetLastError());
+    return LA_OK;
+}
+
+template <typename T>
+static int launch_block_moves(la_ctx *ctx, T *A, int64_t lda, int64_t n, int64_t c_lo,
+                              int64_t c_hi, const int64_t *map, uint64_t *perm)
+{
+    const int64_t ncols = c_lo + (n - c_hi);
+    if (ncols <= 0 && !perm) return LA_OK;
+    constexpr int64_t LPR = 128 / sizeof(T);
+    ProfScope ps(ctx, LA_K_ROWMOVE, 0.0, 2.0 * BLK_MAP_MAX * ncols * sizeof(T));
+    // one extra workgroup permutes the perm vector
+    hipLaunchKernelGGL(k_block_rowmoves<T>, dim3((unsigned)(ceil_div(ncols, LPR) + (perm ? 1 : 0))),
+                       dim3(256), 0, ctx->stream, A, lda, (int)n, (int)c_lo, (int)c_hi, map, perm);
+    LA_HIP_CHECK(ctx, hipGetLastError());
+    return LA_OK;
 }
 
 // ------------------------------------------------ look-ahead streams
@@ -1328,31 +1373,61 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     // outer block from which the look-ahead schedule runs (kmax: never)
     const LookAhead *la = ext_ws ? nullptr : lookahead_streams(ctx);
     int64_t K0la = kmax;
-    if (la)
-        for (int64_t K0 = 0; K0 + NB_OUT < kmax && K0 + NB_OUT < n; K0 += NB_OUT)
-            if (masked_panel_rpl<T>((int)(m - K0), la->panel_cus) > 0) { K0la = K0; break; }
+    // Which blocks go to the column-distributed kernel: by their rows alone,
+    // so that every schedule and entry point factors a block the same way.
+    // Not the factor of a matrix of at most NB_IN columns that one workgroup
+    // holds (it keeps the reference's operation order), nor the factors with
+    // rounded update operands, whose in-block updates round as well.
+    const bool lp = upd_prec == LA_PREC_BF16 || upd_prec == LA_PREC_FP16;
+    const bool exact = kmax <= NB_IN && (size_t)m * (kmax + 1) * sizeof(T) <= 96 * 1024;
+    T *pub = nullptr;
+    const int num_cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    auto block_for = [&](int64_t K0) -> const BlockCfg * {
+        return pub ? block_cfg<T>(m - K0, num_cus) : nullptr;
+    };
     // panel workspace
     size_t slot_bytes = (size_t)2 * PANEL_MAXP * CAND_WORDS * sizeof(uint64_t);
     size_t row_bytes = 256;
     size_t diag_bytes = (size_t)2 * 2 * NB_IN * sizeof(uint64_t);
     size_t map_bytes = (size_t)(1 + 4 * NB_IN) * sizeof(int64_t);
+    size_t bmap_bytes = (size_t)(1 + 2 * BLK_MAP_MAX) * sizeof(int64_t);
     constexpr int RING = 2 * (NB_OUT / NB_IN);           // swap maps of two blocks
     auto al = [](size_t x) { return ws_align(x); };
+    static_assert(RING / 2 * ((1 + 4 * NB_IN) * 8) >= (1 + 2 * BLK_MAP_MAX) * 8,
+                  "a block's map fits the place of its panels' maps");
     void *base = ext_ws;
     int st;
     // look-ahead: swap maps and L11^-1 blocks of two outer blocks, since the
     // update stream still applies block j (row moves, U12) while the panel
     // stream factors block j+1
     const size_t linv_bytes = al((size_t)(NB_OUT / NB_IN) * NB_IN * NB_IN * sizeof(T));
-    const size_t ring_bytes = K0la < kmax ? RING * al(map_bytes) + linv_bytes : 0;
+    const size_t ring_bytes = la ? RING * al(map_bytes) + linv_bytes : 0;
     if (!base && (st = ws_get(ctx, WS_PANEL, panel_ws_bytes(sizeof(T)) + ring_bytes, &base)))
         return st;
+    // the published multipliers; without room for them the row-distributed
+    // panels factor every block
+    if (!lp && !exact && block_cfg<T>(m - (kmax - 1) / NB_OUT * NB_OUT, num_cus)) {
+        if (ext_ws)
+            pub = (T *)((char *)ext_ws + NOALLOC_PUB_OFF);
+        else
+            pub = (T *)ws_try(ctx, WS_PUB, BLK_PUB_BYTES);
+    }
+    if (la)
+        for (int64_t K0 = 0; K0 + NB_OUT < kmax && K0 + NB_OUT < n; K0 += NB_OUT) {
+            const BlockCfg *bc = block_for(K0);
+            if (bc ? NB_OUT / bc->cw <= la->panel_cus
+                   : masked_panel_rpl<T>((int)(m - K0), la->panel_cus) > 0) {
+                K0la = K0;
+                break;
+            }
+        }
     PanelWS pw;
     char *b = (char *)base;
     pw.slots = (uint64_t *)b; b += al(slot_bytes);
     pw.rowbuf = b; b += al(row_bytes);
     pw.diagbuf = b; b += al(diag_bytes);
-    pw.swapmap = (int64_t *)b; b += al(map_bytes);
+    pw.swapmap = (int64_t *)b; b += al(bmap_bytes);
+    uint64_t *pv = (uint64_t *)b; b += al((size_t)NB_OUT * sizeof(uint64_t));
     T *linv_ring = (T *)b;
     b += linv_bytes;
     int64_t *swap_ring = (int64_t *)b;
@@ -1364,6 +1439,7 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     if ((st = fill_u64(ctx, pw.slots, nslot_words, 0xffffffff00000000ull))) return st;
     if ((st = fill_u64(ctx, (uint64_t *)pw.diagbuf, 2 * 2 * NB_IN, 0xffffffff00000000ull)))
         return st;
+    if (pub && (st = fill_u64(ctx, pv, NB_OUT, 0xffffffff00000000ull))) return st;
     if ((st = fill_i32(ctx, d_status, 1, 0))) return st;
     if (d_perm && (st = iota_u64(ctx, d_perm, m))) return st;
     const uint64_t ticks = spin_limit_ticks(ctx);
@@ -1433,7 +1509,16 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     // plain schedule
     for (int64_t K0 = 0; K0 < K0la; K0 += NB_OUT) {
         const int64_t nbo = std::min<int64_t>(NB_OUT, kmax - K0);
-        if ((st = factor_block(K0, nbo, pw.swapmap, 0, linv_ring, 0, true))) return st;
+        if (const BlockCfg *bc = block_for(K0)) {
+            if ((st = launch_block<T>(ctx, *bc, A + K0 * lda + K0, lda, (int)(m - K0), (int)nbo,
+                                      (int)K0, d_ipiv, pub, pv, pw.swapmap, d_status, ticks,
+                                      linv_ring)))
+                return st;
+            if ((st = launch_block_moves<T>(ctx, A, lda, n, K0, K0 + nbo, pw.swapmap, d_perm)))
+                return st;
+        } else if ((st = factor_block(K0, nbo, pw.swapmap, 0, linv_ring, 0, true))) {
+            return st;
+        }
         if (n - (K0 + nbo) > 0) {
             if ((st = block_u12(K0, nbo, K0 + nbo, n - (K0 + nbo), linv_ring))) return st;
             if ((st = block_gemm(K0, nbo, K0 + nbo, n - (K0 + nbo)))) return st;
@@ -1477,7 +1562,10 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
         const int npan = (int)ceil_div(nbo, (int64_t)NB_IN);
         sw.use(la->panel);
         if (K0 > K0la) LA_HIP_CHECK(ctx, hipStreamWaitEvent(la->panel, ev_la, 0));
-        if ((st = factor_block(K0, nbo, maps, ring_stride, linvs, la->panel_cus, false)))
+        const BlockCfg *bc = block_for(K0);
+        if (bc ? (st = launch_block<T>(ctx, *bc, A + K0 * lda + K0, lda, (int)(m - K0), (int)nbo,
+                                       (int)K0, d_ipiv, pub, pv, maps, d_status, ticks, linvs))
+               : (st = factor_block(K0, nbo, maps, ring_stride, linvs, la->panel_cus, false)))
             return st;
         LA_HIP_CHECK(ctx, hipEventRecord(ev_pan, la->panel));
         const bool shared_prev = share_pending;
@@ -1497,16 +1585,18 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
         const int64_t c1 = K0 + nbo, ncol = n - c1;
         const int64_t nla = std::min<int64_t>(NB_OUT, std::max<int64_t>(ncol, 0));
         if (nla > 0) {
-            if ((st = launch_rowmoves<T>(ctx, A + c1, lda, nla, 0, 0, maps, nullptr, npan,
-                                         (int64_t)ring_stride)))
+            if (bc ? (st = launch_block_moves<T>(ctx, A + c1, lda, nla, 0, 0, maps, nullptr))
+                   : (st = launch_rowmoves<T>(ctx, A + c1, lda, nla, 0, 0, maps, nullptr, npan,
+                                              (int64_t)ring_stride)))
                 return st;
             if ((st = block_u12(K0, nbo, c1, nla, linvs))) return st;
             if ((st = block_gemm(K0, nbo, c1, nla))) return st;
         }
         LA_HIP_CHECK(ctx, hipEventRecord(ev_la, la->update));
         if (shared_prev) LA_HIP_CHECK(ctx, hipStreamWaitEvent(la->update, ev_share, 0));
-        if ((st = launch_rowmoves<T>(ctx, A, lda, n, K0, c1 + nla, maps, d_perm, npan,
-                                     (int64_t)ring_stride)))
+        if (bc ? (st = launch_block_moves<T>(ctx, A, lda, n, K0, c1 + nla, maps, d_perm))
+               : (st = launch_rowmoves<T>(ctx, A, lda, n, K0, c1 + nla, maps, d_perm, npan,
+                                          (int64_t)ring_stride)))
             return st;
         if ((st = block_u12(K0, nbo, c1 + nla, ncol - nla, linvs))) return st;
         const int64_t nbulk = ncol - nla, rows = m - c1;
@@ -2101,9 +2191,6 @@ template int getrf_core<float>(la_ctx *, int64_t, int64_t, float *, int64_t, int
 // the process ends.  Its device address is looked up once per device (in
 // la_ctx_create, with that device current) and kept in g_scratch_ptr; host
 // code uses only that address, never the array's name.
-constexpr int64_t NOALLOC_MAX_K = 65536;
-constexpr size_t NOALLOC_PANEL_BYTES = panel_ws_bytes(sizeof(double));
-constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PANEL_BYTES + NOALLOC_MAX_K * sizeof(int64_t);
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static void *g_scratch_ptr[NOALLOC_MAX_DEVICES];

@@ -71,7 +71,7 @@ struct la_ctx {
     int64_t hbm_bytes = 0;
     int clock_khz = 0;
     int64_t ws_limit = 0;
-    lahip::Workspace ws[9];     // independent grow-only workspaces (WS_* ids)
+    lahip::Workspace ws[10];    // independent grow-only workspaces (WS_* ids)
     int32_t *d_scratch = nullptr;   // 4 KiB of device status/counter words
     int32_t *h_pinned = nullptr;    // 4 KiB pinned host mirror
     std::string last_error;
@@ -97,7 +97,7 @@ namespace lahip {
 // invalidates earlier pointers from the SAME slot, so each slot has one user
 // per API call.
 enum { WS_HOST = 0, WS_PANEL = 1, WS_SYNC = 2, WS_PIV = 3, WS_LP = 4, WS_IR = 5,
-       WS_BATCH = 6, WS_GEN = 7, WS_QR = 8, WS_COUNT = 9 };
+       WS_BATCH = 6, WS_GEN = 7, WS_QR = 8, WS_PUB = 9, WS_COUNT = 10 };
 
 // Device scratch words (ctx->d_scratch, 1024 int32):
 //   [0]  sticky device error (LA_ERR_TIMEOUT from bounded waits)
@@ -112,6 +112,10 @@ int read_scratch(la_ctx *ctx, const int32_t *d, int32_t *h, int n);
 int check_sticky(la_ctx *ctx);
 // Returns a device buffer of at least `bytes` from workspace slot `id`.
 int ws_get(la_ctx *ctx, int id, size_t bytes, void **out);
+// As ws_get, but for an optional buffer: null (and no error) when the
+// workspace limit or the device has no room for it.  WS_PUB is such a slot:
+// ws_get gives it back when another slot needs its room under the limit.
+void *ws_try(la_ctx *ctx, int id, size_t bytes);
 
 #define LA_HIP_CHECK(ctx, expr)                                         \
     do {                                                                \
