@@ -1218,7 +1218,8 @@ static int trail_gemm(la_ctx *ctx, int upd_prec, int64_t M, int64_t N, int64_t K
         if (upd_prec == LA_PREC_BF16 || upd_prec == LA_PREC_FP16)
             return gemm_lp(ctx, upd_prec, M, N, K, -1.f, A, lda, B, ldb, 1.f, C, ldc);
     }
-    return gemm_rm<T>(ctx, M, N, K, T(-1), A, lda, B, ldb, T(1), C, ldc, false, false);
+    // no K split: the schedules cut an update's columns differently and agree bit for bit
+    return gemm_rm<T>(ctx, M, N, K, T(-1), A, lda, B, ldb, T(1), C, ldc, false, false, false);
 }
 
 // Panel workspace of getrf_core: exchange slots, row buffer, diagonal-row

@@ -151,11 +151,13 @@ int check_diag_zero(la_ctx *ctx, int64_t n, const double *LU, int64_t ld, int32_
 // ---- kernel launchers implemented in the .hip translation units ----------
 // GEMM: C = alpha*A*op(B) + beta*C, row-major.  trans_b: B is given as an
 // N x K row-major matrix (B^T).  lower_only: skip tiles strictly above the
-// diagonal (symmetric rank-k updates).
+// diagonal (symmetric rank-k updates).  split_k: the sum over k may be split
+// by a rule that looks at M and N too; without it an element's value does not
+// depend on which rows and columns are computed in the same call.
 template <typename T>
 int gemm_rm(la_ctx *ctx, int64_t M, int64_t N, int64_t K, T alpha,
             const T *A, int64_t lda, const T *B, int64_t ldb, T beta,
-            T *C, int64_t ldc, bool trans_b, bool lower_only);
+            T *C, int64_t ldc, bool trans_b, bool lower_only, bool split_k = true);
 
 // Blocked right-looking LU with partial pivoting in precision T, in place.
 // d_ipiv (device, min(m,n)) receives LAPACK-style swaps (row k exchanged
