@@ -9,7 +9,9 @@
 //      panel lives in registers (4 rows per thread, one barrier per column,
 //      candidates exchanged through LDS), its row interchanges are applied to
 //      the other columns as one permutation of at most 2*NB rows, then
-//      U12 = L11^-1 A12 and the trailing update A22 -= L21 U12 on MFMA;
+//      U12 = L11^-1 A12 and the update A22 -= L21 U12 on MFMA: of the rest
+//      of a 64-column outer block after each panel, of everything to its
+//      right once the outer block is done;
 //   3. refinement: x = 0, then repeat { r = b - A x in FP64 from A_i;
 //      eta = max_c ||r_c|| / (||A|| ||x_c|| + ||b_c||); stop when eta <= tol;
 //      solve L U d = P r in working precision (vector in LDS); x += d }.
@@ -23,33 +25,40 @@
 // Each problem is LUDecomposition::new + solve (src/decomp/lu.rs:104-278)
 // in structure; pivots follow the reference's rule (largest |v|, lowest row
 // on ties) in the working precision.
-#include "la_common.hpp"
+//
+// What bounds it: 4096 problems, n log-uniform in [32, 1024], 1-8 right-hand
+// sides, take 23.1 ms in FP32 (FP64 28.5, FP16 39.3; 57, 61.5 and 136 before
+// the products with few columns went to MFMA, panels to blocks of eight
+// columns and updates to outer blocks of 64).  Of the FP32 time the updates
+// are 6.4 ms, panels 4.5, substitution 3.4 and residuals 3.0 (each reads its
+// matrix once at about 5 TB/s), conversion 2.0, row moves 2.1, U12 1.5.
+#include "lu_device.hpp"
 #include <cmath>
+#include <utility>
 
 namespace lahip {
 
 constexpr int BL_MAXN = 1024;
 constexpr int BL_NT = 256;
 constexpr int BL_SLOTS = BL_MAXN / BL_NT;   // panel rows per thread
-constexpr int BL_CHUNK = BL_NT;             // columns per TRSM + update chunk
-constexpr int BL_MVC = 64;                  // columns per row-move chunk
+constexpr int BL_KO = 64;                   // outer block: rank of the trailing update
 constexpr int BL_MAXRHS = 8;
 constexpr int BL_Y_BYTES = 32768;           // right-hand-side block in LDS
-constexpr int BL_STG_BYTES = 36864;         // U12 chunk / row-move staging
+constexpr int BL_STG_BYTES = 36864;         // U12 chunk, x block or diagonal tile
 constexpr int BL_BIG = 1 << 30;             // position of an absent row
 
 template <int MODE> struct BlCfg;
 template <> struct BlCfg<LA_PREC_FP64> {
     typedef double T; typedef double E;
-    static constexpr int NB = 16, PAD = 1;
+    static constexpr int NB = 16;
 };
 template <> struct BlCfg<LA_PREC_FP32> {
     typedef float T; typedef float E;
-    static constexpr int NB = 32, PAD = 4;
+    static constexpr int NB = 32;
 };
 template <> struct BlCfg<LA_PREC_FP16> {
     typedef float T; typedef _Float16 E;
-    static constexpr int NB = 32, PAD = 8;
+    static constexpr int NB = 32;
 };
 
 // pivot key: |v| bits + 1, NaN -> 0 (never preferred over a number)
@@ -61,14 +70,43 @@ __device__ inline uint64_t bl_key(double v) {
     const uint64_t b = (uint64_t)__double_as_longlong(v) & 0x7fffffffffffffffull;
     return b > 0x7ff0000000000000ull ? 0ull : b + 1ull;
 }
-__device__ inline uint64_t bl_shfl_xor_u64(uint64_t v, int m) {
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), m);
-    return ((uint64_t)hi << 32) | lo;
-}
 // (key, q) lexicographic with q = ~position: larger |v| first, lower row on ties
 __device__ inline bool bl_better(uint64_t k1, uint32_t q1, uint64_t k0, uint32_t q0) {
     return k1 > k0 || (k1 == k0 && q1 > q0);
+}
+// The wavefront's largest (key, q), to every lane: DPP maxima of the key's
+// high word (FP32: of the whole key); lower words and q only among several
+// lanes at that maximum.
+__device__ inline uint32_t bl_pick_u32(uint32_t v, uint64_t hit) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v,
+                                               __ffsll((unsigned long long)hit) - 1);
+}
+template <typename T> __device__ inline void bl_wave_best(uint64_t &key, uint32_t &q) {
+    uint32_t hi = (uint32_t)(key >> 32), lo = (uint32_t)key;
+    uint64_t hit;
+    if (sizeof(T) == 8) {
+        const uint32_t mhi = wave_max_u32(hi);
+        hit = __ballot(hi == mhi);
+        hi = mhi;
+        uint32_t mlo = bl_pick_u32(lo, hit);
+        if (__popcll(hit) > 1) {
+            mlo = wave_max_u32((hit >> (threadIdx.x & 63)) & 1 ? lo : 0u);
+            hit &= __ballot(lo == mlo);
+        }
+        lo = mlo;
+    } else {                        // keys below 2^32
+        const uint32_t mlo = wave_max_u32(lo);
+        hit = __ballot(lo == mlo);
+        lo = mlo;
+    }
+    uint32_t mq = bl_pick_u32(q, hit);
+    if (__popcll(hit) > 1) mq = wave_max_u32((hit >> (threadIdx.x & 63)) & 1 ? q : 0u);
+    key = ((uint64_t)hi << 32) | lo;
+    q = mq;
+}
+template <typename F, int... I>
+__device__ __forceinline__ void bl_for_each(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
 }
 __device__ inline float bl_bcast(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
@@ -90,30 +128,39 @@ __device__ inline double bl_wave_sum(double v) {
     return v;
 }
 
-template <int MODE> struct BlMfma;
-template <> struct BlMfma<LA_PREC_FP64> {
+// FP32 / FP64 MFMA, the accumulator row of its element r, and the K batch of
+// bl_rows_times
+template <typename T> struct BlVec;
+template <> struct BlVec<float> {
+    typedef f4_t acc_t;
+    static constexpr int KB = 128;
+    __device__ static inline acc_t mfma(float a, float b, acc_t c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ static inline int drow(int lhi, int r) { return 4 * lhi + r; }
+};
+template <> struct BlVec<double> {
+    typedef d4_t acc_t;
+    static constexpr int KB = 64;
+    __device__ static inline acc_t mfma(double a, double b, acc_t c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
     __device__ static inline int drow(int lhi, int r) { return lhi + 4 * r; }
-};
-template <> struct BlMfma<LA_PREC_FP32> {
-    __device__ static inline int drow(int lhi, int r) { return 4 * lhi + r; }
-};
-template <> struct BlMfma<LA_PREC_FP16> {
-    __device__ static inline int drow(int lhi, int r) { return 4 * lhi + r; }
 };
 
 // LDS of one workgroup (about 77 KB: two workgroups fit a CU)
 template <int MODE> struct BlLds {
     typedef typename BlCfg<MODE>::T T;
     static constexpr int NB = BlCfg<MODE>::NB;
-    __align__(16) unsigned char y[BL_Y_BYTES];       // RHS block, T[n][g]
-    __align__(16) unsigned char stg[BL_STG_BYTES];   // E[BL_CHUNK][NB+PAD] or T[2NB][BL_MVC]
-    T l11[NB][NB + 1];
+    __align__(16) unsigned char y[BL_Y_BYTES];       // RHS block, T[n][g], or L11
+    __align__(16) unsigned char stg[BL_STG_BYTES];   // U chunk, x block (double[n][g]) or T[64][65]
     T cand_row[2][4][NB];
     uint64_t cand_key[2][4];
     uint32_t cand_q[2][4];
-    int mv_src[2 * NB], mv_dst[2 * NB], mv_tmp[2 * NB];
+    int mv_src[2 * NB], mv_dst[2 * NB];
     int nmv, prob, singular;
     double red[4 * 2 * BL_MAXRHS];
+    double bn[BL_MAXRHS], xn[BL_MAXRHS], rn[BL_MAXRHS];   // max |b_c|, |x_c|, |r_c|
 };
 
 // ---------------------------------------------------------------- convert
@@ -155,20 +202,36 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
 {
     typedef typename BlCfg<MODE>::T T;
     typedef typename BlCfg<MODE>::E E;
-    constexpr int NB = BlCfg<MODE>::NB, PAD = BlCfg<MODE>::PAD;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    typedef typename BlVec<T>::acc_t acc_t;
+    // columns per U12 chunk, its LDS stride, K per MFMA group, column tiles
+    // per step.  Strides keep the four lane groups of a fragment read in
+    // different LDS banks.
+    constexpr int CC = MODE == LA_PREC_FP64 ? 64 : MODE == LA_PREC_FP32 ? 128 : 256;
+    constexpr int US = MODE == LA_PREC_FP16 ? BL_KO + 8 : CC + 4;
+    constexpr int KS = MODE == LA_PREC_FP16 ? 32 : 16, G = sizeof(T) == 8 ? 4 : 8;
+    static_assert((MODE == LA_PREC_FP16 ? CC : BL_KO) * US * sizeof(E) <= BL_STG_BYTES, "U chunk");
+    static_assert(BL_KO * BL_KO * sizeof(T) <= BL_Y_BYTES, "L11");
+    E *const ustg = reinterpret_cast<E *>(L.stg);
+    constexpr int NB = BlCfg<MODE>::NB, NBLK = NB / 8;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lhi = lane >> 4;
     const float uinv = 1.0f / uscale;
     if (tid == 0) L.singular = 0;
 
     for (int k0 = 0; k0 < n; k0 += NB) {
         const int jb = min(NB, n - k0), m = n - k0;
+        const int K0 = k0 / BL_KO * BL_KO, kend = min(n, K0 + BL_KO);   // outer block
         T *Wp = W + (int64_t)k0 * n + k0;
         // ---- panel: rows k0..n-1, columns k0..k0+jb-1, in registers.
-        // The column being eliminated is always a[.][0]: after each step the
-        // row arrays rotate left by one (the finished multiplier moves to the
-        // end), so the column loop is not unrolled and every register index
-        // stays static; NB rotations restore the original column order.
+        // The column being eliminated is register c of the first block of
+        // eight; after eight columns the row arrays rotate left by one block
+        // (a finished block moves to the end), so the code is eight columns
+        // long, every register index stays static, and only the blocks that
+        // still hold active columns are updated.  NB / 8 rotations restore
+        // the original column order.  (One column per step with a rotation
+        // each and a shuffle tree for the pivot: 10.5 of the 33 ms of 4096
+        // FP32 problems, n in [32, 1024]; now 4.5.)
         T a[BL_SLOTS][NB];
         int pos[BL_SLOTS];
 #pragma unroll
@@ -184,77 +247,98 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
                 if (!(r < m && c < jb)) a[s][c] = (T)0;
         }
         if (tid == 0) L.nmv = 0;
-#pragma unroll 1
-        for (int j = 0; j < NB; ++j) {
-            if (j < jb) {
-                const int par = j & 1;
-                uint64_t bk = 0;
-                uint32_t bq = 0;
+        auto column = [&](auto c_c, int it) __attribute__((always_inline)) {
+            constexpr int c0 = decltype(c_c)::value;
+            const int j = 8 * it + c0;
+            if (j >= jb) return;                        // uniform
+            const int par = j & 1;
+            // largest key of the thread's rows, lowest position on ties
+            uint64_t bk = 0;
+            uint32_t bq = 0;
 #pragma unroll
-                for (int s = 0; s < BL_SLOTS; ++s)
-                    if (pos[s] >= j && pos[s] < m) {
-                        const uint64_t kk = bl_key(a[s][0]);
-                        const uint32_t qq = ~(uint32_t)pos[s];
-                        if (bl_better(kk, qq, bk, bq)) { bk = kk; bq = qq; }
-                    }
-#pragma unroll
-                for (int msk = 32; msk >= 1; msk >>= 1) {
-                    const uint64_t ok = bl_shfl_xor_u64(bk, msk);
-                    const uint32_t oq = (uint32_t)__shfl_xor((int)bq, msk);
-                    if (bl_better(ok, oq, bk, bq)) { bk = ok; bq = oq; }
+            for (int s = 0; s < BL_SLOTS; ++s)
+                if (pos[s] >= j && pos[s] < m) {
+                    const uint64_t kk = bl_key(a[s][c0]);
+                    const uint32_t qq = ~(uint32_t)pos[s];
+                    if (bl_better(kk, qq, bk, bq)) { bk = kk; bq = qq; }
                 }
-                const int wpos = (int)~bq;
+            bl_wave_best<T>(bk, bq);
+            const int wpos = (int)~bq;
 #pragma unroll
-                for (int s = 0; s < BL_SLOTS; ++s)
-                    if (pos[s] == wpos && bq != 0) {
+            for (int s = 0; s < BL_SLOTS; ++s)
+                if (pos[s] == wpos && bq != 0) {
 #pragma unroll
-                        for (int c = 0; c < NB; ++c) L.cand_row[par][wave][c] = a[s][c];
-                    }
-                if (lane == 0) { L.cand_key[par][wave] = bk; L.cand_q[par][wave] = bq; }
-                __syncthreads();
-                uint64_t gk = L.cand_key[par][0];
-                uint32_t gq = L.cand_q[par][0];
-                int gw = 0;
+                    for (int b = 0; b < NBLK; ++b)
+                        if (b < NBLK - it) {
 #pragma unroll
-                for (int w = 1; w < 4; ++w) {
-                    const uint64_t k2 = L.cand_key[par][w];
-                    const uint32_t q2 = L.cand_q[par][w];
-                    if (bl_better(k2, q2, gk, gq)) { gk = k2; gq = q2; gw = w; }
+                            for (int c = 8 * b; c < 8 * b + 8; ++c)
+                                L.cand_row[par][wave][c] = a[s][c];
+                        }
                 }
-                const int ppos = (int)~gq;      // current position of the pivot row
-                // pivot row: active columns only (the tail holds its multipliers)
-                T prow[NB];
+            if (lane == 0) { L.cand_key[par][wave] = bk; L.cand_q[par][wave] = bq; }
+            __syncthreads();
+            uint64_t gk = L.cand_key[par][0];
+            uint32_t gq = L.cand_q[par][0];
+            int gw = 0;
 #pragma unroll
-                for (int c = 0; c < NB; ++c) prow[c] = c < NB - j ? L.cand_row[par][gw][c] : (T)0;
-                const T piv = prow[0];
+            for (int w = 1; w < 4; ++w) {
+                const uint64_t k2 = L.cand_key[par][w];
+                const uint32_t q2 = L.cand_q[par][w];
+                if (bl_better(k2, q2, gk, gq)) { gk = k2; gq = q2; gw = w; }
+            }
+            const int ppos = (int)~gq;      // current position of the pivot row
+            const T *prow = L.cand_row[par][__builtin_amdgcn_readfirstlane(gw)];
+            const T piv = prow[c0];
 #pragma unroll
-                for (int s = 0; s < BL_SLOTS; ++s) {
-                    if (pos[s] == ppos) pos[s] = j;
-                    else if (pos[s] == j) pos[s] = ppos;
+            for (int s = 0; s < BL_SLOTS; ++s) {
+                if (pos[s] == ppos) pos[s] = j;
+                else if (pos[s] == j) pos[s] = ppos;
+            }
+            if (!(piv != (T)0)) {           // exact zero (or NaN) pivot: no scaling
+                if (tid == 0) L.singular = 1;
+                return;
+            }
+            const T rinv = (T)1 / piv;
+            T l[BL_SLOTS];
+#pragma unroll
+            for (int s = 0; s < BL_SLOTS; ++s) {
+                l[s] = (T)0;
+                if (pos[s] > j && pos[s] < m) {
+                    l[s] = (MODE == LA_PREC_FP64) ? a[s][c0] / piv : a[s][c0] * rinv;
+                    a[s][c0] = l[s];
                 }
-                if (!(piv != (T)0)) {           // exact zero (or NaN) pivot: no scaling
-                    if (tid == 0) L.singular = 1;
-                } else {
-                    const T rinv = (T)1 / piv;
+            }
+#pragma unroll
+            for (int b = 0; b < NBLK; ++b)
+                if (b < NBLK - it) {
+                    T u[8];
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) u[c] = prow[8 * b + c];
 #pragma unroll
                     for (int s = 0; s < BL_SLOTS; ++s)
                         if (pos[s] > j && pos[s] < m) {
-                            const T l = (MODE == LA_PREC_FP64) ? a[s][0] / piv : a[s][0] * rinv;
 #pragma unroll
-                            for (int c = 1; c < NB; ++c) a[s][c] -= l * prow[c];
-                            a[s][0] = l;
+                            for (int c = 0; c < 8; ++c)
+                                if (8 * b + c > c0) a[s][8 * b + c] -= l[s] * u[c];
                         }
                 }
-            }
+        };
+#pragma unroll 1
+        for (int it = 0; it < NBLK; ++it) {
+            bl_for_each([&](auto c_c) __attribute__((always_inline)) { column(c_c, it); },
+                        std::make_integer_sequence<int, 8>{});
 #pragma unroll
             for (int s = 0; s < BL_SLOTS; ++s) {
-                const T t0 = a[s][0];
+                T t[8];
 #pragma unroll
-                for (int c = 0; c < NB - 1; ++c) a[s][c] = a[s][c + 1];
-                a[s][NB - 1] = t0;
+                for (int c = 0; c < 8; ++c) t[c] = a[s][c];
+#pragma unroll
+                for (int c = 0; c < NB - 8; ++c) a[s][c] = a[s][c + 8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c) a[s][NB - 8 + c] = t[c];
             }
         }
-        // ---- panel write-back at the final positions, L11, move list
+        // ---- panel write-back at the final positions, move list
 #pragma unroll
         for (int s = 0; s < BL_SLOTS; ++s) {
             const int r = tid + BL_NT * s;
@@ -264,10 +348,6 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
 #pragma unroll
                 for (int c = 0; c < NB; ++c)
                     if (c < jb) dst[c] = a[s][c];
-                if (q < jb) {
-#pragma unroll
-                    for (int c = 0; c < NB; ++c) L.l11[q][c] = c < q ? a[s][c] : (T)0;
-                }
                 if (q != r) {
                     const int idx = atomicAdd(&L.nmv, 1);
                     L.mv_src[idx] = r;
@@ -276,139 +356,184 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
             }
         }
         __syncthreads();
-        const int nmv = L.nmv;
-        // ---- the same row permutation on every column outside the panel
+        const int nmv = __builtin_amdgcn_readfirstlane(L.nmv);
+        // ---- the same row permutation on every column outside the panel.
+        // A wave owns 64 columns and holds all moved rows of them (at most
+        // 2 NB) in registers, so its loads are all in flight together and no
+        // barrier parts them from its stores (staged through LDS with two
+        // barriers per 64 columns and one load in flight per thread this
+        // took 6.4 of the 51 ms of 4096 FP32 problems, n in [32, 1024]; now 2.1).
         if (nmv > 0) {
-            T (*mstg)[BL_MVC] = reinterpret_cast<T (*)[BL_MVC]>(L.stg);
             const int outside = n - jb;
-            for (int x0 = 0; x0 < outside; x0 += BL_MVC) {
-                const int cw = min(BL_MVC, outside - x0);
-                for (int e = tid; e < nmv * cw; e += BL_NT) {
-                    const int i = e / cw, cc = e - i * cw;
-                    const int x = x0 + cc, col = x < k0 ? x : x + jb;
-                    mstg[i][cc] = W[(int64_t)(k0 + L.mv_src[i]) * n + col];
-                }
-                __syncthreads();
-                for (int e = tid; e < nmv * cw; e += BL_NT) {
-                    const int i = e / cw, cc = e - i * cw;
-                    const int x = x0 + cc, col = x < k0 ? x : x + jb;
-                    W[(int64_t)(k0 + L.mv_dst[i]) * n + col] = mstg[i][cc];
-                }
-                __syncthreads();
+            for (int x0 = wave * 64; x0 < outside; x0 += BL_NT) {
+                const int x = min(x0 + lane, outside - 1), col = x < k0 ? x : x + jb;
+                T *const wc = W + (int64_t)k0 * n;       // 32-bit offsets: n <= 1024
+                T rv[2 * NB];
+#pragma unroll
+                for (int e0 = 0; e0 < 2 * NB; e0 += 16)
+                    if (e0 < nmv) {
+#pragma unroll
+                        for (int e = e0; e < e0 + 16; ++e)
+                            rv[e] = wc[(uint32_t)(L.mv_src[min(e, nmv - 1)] * n + col)];
+                    }
+#pragma unroll
+                for (int e0 = 0; e0 < 2 * NB; e0 += 16)
+                    if (e0 < nmv) {
+#pragma unroll
+                        for (int e = e0; e < e0 + 16; ++e)
+                            if (e < nmv && x0 + lane < outside)
+                                wc[(uint32_t)(L.mv_dst[e] * n + col)] = rv[e];
+                    }
             }
-            if (tid < nmv) L.mv_tmp[tid] = perm[k0 + L.mv_src[tid]];
+            int pm = 0;
+            if (tid < nmv) pm = perm[k0 + L.mv_src[tid]];
             __syncthreads();
-            if (tid < nmv) perm[k0 + L.mv_dst[tid]] = L.mv_tmp[tid];
+            if (tid < nmv) perm[k0 + L.mv_dst[tid]] = pm;
             __syncthreads();
         }
-        // ---- U12 = L11^-1 A12 and A22 -= L21 U12, in column chunks
-        const int c_begin = k0 + jb;
-        const int R = n - c_begin;
-        E (*ustg)[NB + PAD] = reinterpret_cast<E (*)[NB + PAD]>(L.stg);
-        for (int cc0 = c_begin; cc0 < n; cc0 += BL_CHUNK) {
-            const int cw = min(BL_CHUNK, n - cc0);
-            {
-                const int col = cc0 + tid;
+        // ---- U12 = L11^-1 A12 and A22 -= L21 U12.  After an inner panel: its
+        // own rows, on the columns left of the outer block's end.  After the
+        // outer block: its BL_KO rows, on every column to the right, so that
+        // the trailing matrix is read and written once per BL_KO columns (a
+        // pass per NB columns moved 145 GB for 4096 FP64 problems, 26 ms of 60;
+        // now 36 GB, 10 ms of 28).
+        const bool outer = k0 + jb == kend;
+        const int ka = outer ? K0 : k0, kd = k0 + jb - ka;
+        const int c_lo = k0 + jb, c_hi = outer ? n : kend;
+        if (c_lo >= c_hi) continue;
+        // kd is NB or BL_KO here: a shorter panel has no column to its right
+        T *l11 = reinterpret_cast<T *>(L.y);                 // [BL_KO][BL_KO]
+#pragma unroll
+        for (int i0 = 0; i0 < BL_KO; i0 += NB)
+            if (i0 < kd) {
+                T v[NB / 4];
+#pragma unroll
+                for (int i = 0; i < NB / 4; ++i)
+                    v[i] = W[(uint32_t)((ka + i0 + wave + 4 * i) * n + ka + min(lane, kd - 1))];
+#pragma unroll
+                for (int i = 0; i < NB / 4; ++i) l11[(i0 + wave + 4 * i) * BL_KO + lane] = v[i];
+            }
+        __syncthreads();
+        for (int u0 = c_lo; u0 < c_hi; u0 += BL_NT) {
+            // one column per thread, NB rows at a time: finished rows of the
+            // column come back from memory (the thread's own stores)
+            const bool valid = u0 + tid < c_hi;
+            const int col = min(u0 + tid, c_hi - 1);
+            for (int p = 0; p < kd; p += NB) {
                 T x[NB];
-                const int colc = min(col, n - 1);
 #pragma unroll
-                for (int i = 0; i < NB; ++i) x[i] = W[(int64_t)(k0 + min(i, jb - 1)) * n + colc];
+                for (int i = 0; i < NB; ++i) x[i] = W[(uint32_t)((ka + p + i) * n + col)];
+                for (int q = 0; q < p; q += NB) {
+                    T y[NB];
 #pragma unroll
-                for (int i = 0; i < NB; ++i)
-                    if (!(tid < cw && i < jb)) x[i] = (T)0;
-#pragma unroll
-                for (int i = 1; i < NB; ++i) {
-                    T acc = x[i];
-#pragma unroll
-                    for (int k = 0; k < i; ++k) acc -= L.l11[i][k] * x[k];
-                    x[i] = acc;
-                }
-                if (tid < cw) {
+                    for (int k = 0; k < NB; ++k) y[k] = W[(uint32_t)((ka + q + k) * n + col)];
+                    const T *lp = l11 + p * BL_KO + q;
 #pragma unroll
                     for (int i = 0; i < NB; ++i)
-                        if (i < jb) W[(int64_t)(k0 + i) * n + col] = x[i];
-                }
 #pragma unroll
-                for (int i = 0; i < NB; ++i)
-                    ustg[tid][i] = (MODE == LA_PREC_FP16) ? (E)((float)x[i] * uscale) : (E)x[i];
+                        for (int k = 0; k < NB; ++k) x[i] -= lp[i * BL_KO + k] * y[k];
+                }
+                const T *lp = l11 + p * BL_KO + p;
+#pragma unroll
+                for (int i = 1; i < NB; ++i)
+#pragma unroll
+                    for (int k = 0; k < i; ++k) x[i] -= lp[i * BL_KO + k] * x[k];
+                if (valid) {
+#pragma unroll
+                    for (int i = 0; i < NB; ++i) W[(uint32_t)((ka + p + i) * n + col)] = x[i];
+                }
+            }
+        }
+        __syncthreads();
+        const int rt_n = (n - c_lo + 15) >> 4;
+        for (int cc0 = c_lo; cc0 < c_hi; cc0 += CC) {
+            const int cw = min(CC, c_hi - cc0);
+            // U chunk to LDS, kd x CC (k-major; FP16: column-major, scaled)
+            constexpr int TPR = CC < BL_NT ? CC : BL_NT, RPP = BL_NT / TPR;
+            const int uc = tid % TPR, ur = tid / TPR, ucol = cc0 + min(uc, cw - 1);
+            for (int k = ur; k < kd; k += 16 * RPP) {
+                T v[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    v[i] = W[(uint32_t)((ka + min(k + i * RPP, kd - 1)) * n + ucol)];
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (k + i * RPP < kd) {
+                        if constexpr (MODE == LA_PREC_FP16)
+                            ustg[uc * US + k + i * RPP] = (E)((float)v[i] * uscale);
+                        else
+                            ustg[(k + i * RPP) * US + uc] = v[i];
+                    }
             }
             __syncthreads();
-            // each wave: one 16-row tile at a time against all column tiles of
-            // the chunk, G column tiles per step with their C values loaded
-            // together so that 4*G reads per lane are in flight
-            const int rt_n = (R + 15) >> 4, ct_n = (cw + 15) >> 4;
-            constexpr int G = sizeof(T) == 8 ? 4 : 8;
+            // Each wave: one 16-row tile against the chunk's column tiles, G
+            // at a time, with the C values of a step loaded together from
+            // clamped positions.  Lane group l / 16 takes four (FP16: eight)
+            // consecutive k of every sixteen (32), so L21 loads are 16 bytes
+            // or more.
+            const int ct_n = (cw + 15) >> 4;
             for (int rt = wave; rt < rt_n; rt += 4) {
-                const int row = c_begin + 16 * rt + l16;
-                const bool rok = row < n;
-                // unconditional loads from clamped positions (issued
-                // together); out-of-range elements are replaced by zero
-                const T *lrow = W + (int64_t)min(row, n - 1) * n + k0;
-                h8_t ah;
-                T af[NB / 4];
-                if constexpr (MODE == LA_PREC_FP16) {
-                    T lv[8];
+                const int row0 = c_lo + 16 * rt;
+                const T *const lrow = W + (uint32_t)(min(row0 + l16, n - 1) * n + ka);
+                h8_t ah[BL_KO / 32];
+                T af[BL_KO / 4];
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) lv[e] = lrow[min(8 * lhi + e, jb - 1)];
+                for (int q = 0; q < BL_KO; q += KS)
+                    if (q < kd) {
+                        T lv[KS / 4];
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int k = 8 * lhi + e;
-                        ah[e] = (_Float16)((rok && k < jb) ? lv[e] : 0.0f);
+                        for (int e = 0; e < KS / 4; ++e) lv[e] = lrow[q + lhi * (KS / 4) + e];
+#pragma unroll
+                        for (int e = 0; e < KS / 4; ++e) {
+                            if constexpr (MODE == LA_PREC_FP16) ah[q / KS][e] = (_Float16)lv[e];
+                            else af[q / 4 + e] = lv[e];
+                        }
                     }
-                } else {
-#pragma unroll
-                    for (int s = 0; s < NB / 4; ++s) af[s] = lrow[min(4 * s + lhi, jb - 1)];
-#pragma unroll
-                    for (int s = 0; s < NB / 4; ++s) {
-                        const int k = 4 * s + lhi;
-                        if (!(rok && k < jb)) af[s] = (T)0;
-                    }
-                }
                 for (int ct0 = 0; ct0 < ct_n; ct0 += G) {
                     T cv[G][4];
+                    uint32_t off[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        off[r] = (uint32_t)(min(row0 + BlVec<T>::drow(lhi, r), n - 1) * n);
 #pragma unroll
                     for (int g = 0; g < G; ++g) {
-                        const int col = cc0 + 16 * (ct0 + g) + l16;
+                        const int col = min(cc0 + 16 * (ct0 + g) + l16, c_hi - 1);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int crow = c_begin + 16 * rt + BlMfma<MODE>::drow(lhi, r);
-                            cv[g][r] = (crow < n && col < cc0 + cw) ? W[(int64_t)crow * n + col]
-                                                                    : (T)0;
-                        }
+                        for (int r = 0; r < 4; ++r) cv[g][r] = W[off[r] + (uint32_t)col];
                     }
+                    acc_t acc[G];
+#pragma unroll
+                    for (int g = 0; g < G; ++g) acc[g] = acc_t{0, 0, 0, 0};
+#pragma unroll
+                    for (int q = 0; q < BL_KO; q += KS)
+                        if (q < kd) {
+                            if constexpr (MODE == LA_PREC_FP16) {
+#pragma unroll
+                                for (int g = 0; g < G; ++g)
+                                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                        ah[q / KS],
+                                        *reinterpret_cast<const h8_t *>(
+                                            &ustg[(16 * (ct0 + g) + l16) * US + q + 8 * lhi]),
+                                        acc[g], 0, 0, 0);
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                                    for (int g = 0; g < G; ++g)
+                                        acc[g] = BlVec<T>::mfma(
+                                            af[q / 4 + e],
+                                            ustg[(q + 4 * lhi + e) * US + 16 * (ct0 + g) + l16],
+                                            acc[g]);
+                            }
+                        }
 #pragma unroll
                     for (int g = 0; g < G; ++g) {
-                        const int cl = 16 * (ct0 + g) + l16;     // < BL_CHUNK: ct < 16
-                        T d[4];
-                        if constexpr (MODE == LA_PREC_FP16) {
-                            const h8_t bfv = *reinterpret_cast<const h8_t *>(&ustg[cl][8 * lhi]);
-                            f4_t acc = {0.f, 0.f, 0.f, 0.f};
-                            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bfv, acc, 0, 0, 0);
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) d[r] = acc[r] * uinv;
-                        } else if constexpr (MODE == LA_PREC_FP64) {
-                            d4_t acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                            for (int s = 0; s < NB / 4; ++s)
-                                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(af[s], ustg[cl][4 * s + lhi],
-                                                                           acc, 0, 0, 0);
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) d[r] = acc[r];
-                        } else {
-                            f4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                            for (int s = 0; s < NB / 4; ++s)
-                                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af[s], ustg[cl][4 * s + lhi],
-                                                                           acc, 0, 0, 0);
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) d[r] = acc[r];
-                        }
-                        const int col = cc0 + cl;
+                        const int cl = 16 * (ct0 + g) + l16;
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            const int crow = c_begin + 16 * rt + BlMfma<MODE>::drow(lhi, r);
-                            if (crow < n && col < cc0 + cw)
-                                W[(int64_t)crow * n + col] = cv[g][r] - d[r];
+                            const T d = MODE == LA_PREC_FP16 ? (T)(acc[g][r] * uinv) : acc[g][r];
+                            if (row0 + BlVec<T>::drow(lhi, r) < n && cl < cw)
+                                W[off[r] + (uint32_t)(cc0 + cl)] = cv[g][r] - d;
                         }
                     }
                 }
@@ -416,110 +541,152 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
             __syncthreads();
         }
     }
+}
+
+// ------------------------------------------------ products with few columns
+// acc (16 x 16, MFMA layout) += M X over the columns [j0, j1) of 16 rows of M,
+// row pointer per lane (row l % 16), X (ldx columns per row, g <= 16 of them)
+// in LDS.  Lane group l / 16 takes four consecutive k of every sixteen, so a
+// lane loads 16 or 32 consecutive bytes and the rows' cache lines are read
+// whole; columns of the result past g are never read.  KB elements of a row
+// are loaded while the KB before them are multiplied: these products are
+// bound by the way to memory (M is read once), and four rows at a time with
+// eight 4- or 8-byte loads in flight reached 1.2 (FP64) and 0.5 TB/s (FP32).
+// Four accumulators, one per sixteen columns of a batch, are added at the end.
+template <typename T>
+__device__ __forceinline__ typename BlVec<T>::acc_t
+bl_rows_times(const T *__restrict__ mrow, const T *X, int ldx, int g, int j0, int j1)
+{
+    typedef typename BlVec<T>::acc_t acc_t;
+    constexpr int KB = BlVec<T>::KB, NC = KB / 16;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lhi = lane >> 4;
+    const T *xc = X + min(l16, g - 1);
+    acc_t acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] = acc_t{0, 0, 0, 0};
+    T v[NC][4], w[NC][4];
+    auto load = [&](T (&d)[NC][4], int j) __attribute__((always_inline)) {
+        if (j + KB <= j1) {
+            const T *src = mrow + j + 4 * lhi;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[c][e] = src[16 * c + e];
+        } else {
+            // from clamped positions, then zeroed
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[c][e] = mrow[min(j + 16 * c + 4 * lhi + e, j1 - 1)];
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (j + 16 * c + 4 * lhi + e >= j1) d[c][e] = T(0);
+        }
+    };
+    if (j0 < j1) load(v, j0);
+    for (int j = j0; j < j1; j += KB) {
+        if (j + KB < j1) load(w, j + KB);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (j + 16 * c < j1) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const T x = xc[min(j + 16 * c + 4 * lhi + e, j1 - 1) * ldx];
+                    acc[c & 3] = BlVec<T>::mfma(v[c][e], x, acc[c & 3]);
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[c][e] = w[c][e];
+    }
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
 }
 
 // ------------------------------------------------ triangular solves in LDS
 // Y (n x g, row-major in LDS) <- L^-1 Y (unit lower), then U^-1 Y, with the
-// packed factor in W.  64-row blocks: the off-diagonal part is a 16-lanes-
-// per-row GEMV, the diagonal block is solved by one wave per right-hand side
-// with the block row in registers and readlane broadcasts.
+// packed factor in W.  64-row blocks: the off-diagonal part on MFMA, sixteen
+// rows per wave; the diagonal tile is loaded (coalesced) before it, staged in
+// LDS and solved one row per lane with readlane broadcasts, each wave taking
+// right-hand sides c and c + 4 together so that their chains overlap.  The
+// upper tile's rows are scaled by the reciprocal of their diagonal once, so
+// the chain has no division (unless a reciprocal is not finite).
 template <typename T>
-__device__ void bl_gemv_sub(int n, const T *__restrict__ W, T *Y, int g, int b0, int bs, int j0,
-                            int j1)
+__device__ void bl_trsv_lu(int n, const T *__restrict__ W, T *Y, int g, unsigned char *stg)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sub = lane >> 4, l16 = lane & 15;
-    for (int i0 = wave * 4; i0 < bs; i0 += 16) {
-        const int il = i0 + sub;
-        const int i = b0 + il;
-        T acc[BL_MAXRHS];
-#pragma unroll
-        for (int c = 0; c < BL_MAXRHS; ++c) acc[c] = (T)0;
-        if (il < bs) {
-            const T *wr = W + (int64_t)i * n;
-#pragma unroll 8
-            for (int j = j0 + l16; j < j1; j += 16) {
-                const T w = wr[j];
-#pragma unroll
-                for (int c = 0; c < BL_MAXRHS; ++c)
-                    if (c < g) acc[c] += w * Y[j * g + c];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < BL_MAXRHS; ++c) {
-            if (c < g) {
-#pragma unroll
-                for (int msk = 8; msk >= 1; msk >>= 1) acc[c] += __shfl_xor(acc[c], msk);
-            }
-        }
-        if (il < bs && l16 == 0) {
-#pragma unroll
-            for (int c = 0; c < BL_MAXRHS; ++c)
-                if (c < g) Y[i * g + c] -= acc[c];
-        }
-    }
-}
-
-template <typename T>
-__device__ void bl_trsv_lu(int n, const T *__restrict__ W, T *Y, int g)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // forward: unit lower
-    for (int b0 = 0; b0 < n; b0 += 64) {
-        const int bs = min(64, n - b0);
-        if (b0 > 0) {
-            bl_gemv_sub<T>(n, W, Y, g, b0, bs, 0, b0);
-            __syncthreads();
-        }
-        for (int c = wave; c < g; c += 4) {
-            const int i = lane;
-            T lrow[64];
-            // unconditional loads from clamped positions, then zeroed
-            const T *wr = W + (int64_t)(b0 + min(i, bs - 1)) * n + b0;
-#pragma unroll
-            for (int k = 0; k < 64; ++k) lrow[k] = wr[min(k, bs - 1)];
-#pragma unroll
-            for (int k = 0; k < 64; ++k)
-                if (!(i < bs && k < i)) lrow[k] = (T)0;
-            T y = i < bs ? Y[(b0 + i) * g + c] : (T)0;
-#pragma unroll
-            for (int k = 0; k < 63; ++k) {
-                if (k + 1 < bs) {
-                    const T yk = bl_bcast(y, k);
-                    if (i > k) y -= lrow[k] * yk;
-                }
-            }
-            if (i < bs) Y[(b0 + i) * g + c] = y;
-        }
-        __syncthreads();
-    }
-    // backward: upper with diagonal
+    T (*D)[65] = reinterpret_cast<T (*)[65]>(stg);
+    static_assert(sizeof(T) * 64 * 65 <= BL_STG_BYTES, "diagonal tile");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lhi = lane >> 4;
     const int nblk = (n + 63) / 64;
-    for (int bi = nblk - 1; bi >= 0; --bi) {
-        const int b0 = bi * 64, bs = min(64, n - b0);
-        if (b0 + bs < n) {
-            bl_gemv_sub<T>(n, W, Y, g, b0, bs, b0 + bs, n);
-            __syncthreads();
+    for (int step = 0; step < 2 * nblk; ++step) {
+        const bool fwd = step < nblk;
+        const int b0 = 64 * (fwd ? step : 2 * nblk - 1 - step), bs = min(64, n - b0);
+        T dv[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int r = (tid >> 6) + 4 * q;
+            dv[q] = W[(int64_t)(b0 + min(r, bs - 1)) * n + b0 + min(lane, bs - 1)];
         }
-        for (int c = wave; c < g; c += 4) {
-            const int i = lane;
-            T urow[64];
-            const T *wr = W + (int64_t)(b0 + min(i, bs - 1)) * n + b0;
+        const int j0 = fwd ? 0 : b0 + bs, j1 = fwd ? b0 : n;
+        if (j0 < j1) {
+            const T *mrow = W + (int64_t)(b0 + min(16 * wave + l16, bs - 1)) * n;
+            const auto acc = bl_rows_times<T>(mrow, Y, g, g, j0, j1);
 #pragma unroll
-            for (int k = 0; k < 64; ++k) urow[k] = wr[min(k, bs - 1)];
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * wave + BlVec<T>::drow(lhi, r);
+                if (i < bs && l16 < g) Y[(b0 + i) * g + l16] -= acc[r];
+            }
+        }
 #pragma unroll
-            for (int k = 0; k < 64; ++k)
-                if (!(i < bs && k >= i && k < bs)) urow[k] = (T)1;
-            T y = i < bs ? Y[(b0 + i) * g + c] : (T)0;
+        for (int q = 0; q < 16; ++q) D[(tid >> 6) + 4 * q][lane] = dv[q];
+        __syncthreads();
+        if (wave < g) {
+            const int i = min(lane, bs - 1);
+            const bool two = wave + 4 < g;
+            T *y0p = Y + (b0 + i) * g + wave, *y1p = y0p + (two ? 4 : 0);
+            T y0 = *y0p, y1 = *y1p;
+            T row[64];
 #pragma unroll
-            for (int k = 63; k >= 0; --k) {
-                if (k < bs) {
-                    if (i == k) y = y / urow[k];
-                    const T yk = bl_bcast(y, k);
-                    if (i < k) y -= urow[k] * yk;
+            for (int k = 0; k < 64; ++k) row[k] = D[i][k];
+            if (fwd) {
+#pragma unroll
+                for (int k = 0; k < 63; ++k)
+                    if (k + 1 < bs) {
+                        const T a = bl_bcast(y0, k), b = bl_bcast(y1, k);
+                        const T l = i > k ? row[k] : (T)0;
+                        if (i > k) { y0 -= l * a; y1 -= l * b; }
+                    }
+            } else {
+                const T d = D[i][i], rd = (T)1 / d;
+                if (!__any(!(fabs(rd) < (T)INFINITY))) {
+                    y0 *= rd;
+                    y1 *= rd;
+#pragma unroll
+                    for (int k = 0; k < 64; ++k) row[k] *= rd;
+#pragma unroll
+                    for (int k = 63; k >= 1; --k)
+                        if (k < bs) {
+                            const T a = bl_bcast(y0, k), b = bl_bcast(y1, k);
+                            if (i < k) { y0 -= row[k] * a; y1 -= row[k] * b; }
+                        }
+                } else {
+#pragma unroll 1
+                    for (int k = bs - 1; k >= 0; --k) {
+                        if (i == k) { y0 = y0 / d; y1 = y1 / d; }
+                        const T a = bl_bcast(y0, k), b = bl_bcast(y1, k), u = D[i][k];
+                        if (i < k) { y0 -= u * a; y1 -= u * b; }
+                    }
                 }
             }
-            if (i < bs) Y[(b0 + i) * g + c] = y;
+            if (lane < bs) {
+                *y0p = y0;
+                if (two) *y1p = y1;
+            }
         }
         __syncthreads();
     }
@@ -527,18 +694,19 @@ __device__ void bl_trsv_lu(int n, const T *__restrict__ W, T *Y, int g)
 
 // ----------------------------------------------------------- refinement
 // r = b - A x (FP64) for the rows in pivot order; Y[i][c] = r[perm[i]][c]
-// in working precision; rn[c] = max |r_c| (all threads get it).
+// in working precision; L.rn[c] = max |r_c|.  Sixteen rows per wave at a time
+// on FP64 MFMA.
 template <int MODE>
 __device__ void bl_residual(int n, int nrhs, int c0, int g, bool first,
                             const double *__restrict__ Ap, const double *__restrict__ Bp,
-                            const double *Xp, const int *__restrict__ perm, BlLds<MODE> &L,
-                            double *rn)
+                            const double *Xp, const int *__restrict__ perm, BlLds<MODE> &L)
 {
     typedef typename BlCfg<MODE>::T T;
     T *Y = reinterpret_cast<T *>(L.y);
     double *xs = reinterpret_cast<double *>(L.stg);      // x block, [j][g], in LDS
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sub = lane >> 4, l16 = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lhi = lane >> 4;
     if (!first) {
         for (int e = tid; e < n * g; e += BL_NT) {
             const int j = e / g, c = e - j * g;
@@ -546,66 +714,42 @@ __device__ void bl_residual(int n, int nrhs, int c0, int g, bool first,
         }
         __syncthreads();
     }
-    double rmax[BL_MAXRHS];
+    double rmax = 0.0;                                   // of column l16
+    for (int i0 = wave * 16; i0 < n; i0 += 64) {
+        // right-hand sides of the rows this lane ends up with
+        double bv[4];
 #pragma unroll
-    for (int c = 0; c < BL_MAXRHS; ++c) rmax[c] = 0.0;
-    for (int i0 = wave * 4; i0 < n; i0 += 16) {
-        const int i = i0 + sub;
-        double acc[BL_MAXRHS];
+        for (int r = 0; r < 4; ++r)
+            bv[r] = Bp[(int64_t)perm[min(i0 + BlVec<double>::drow(lhi, r), n - 1)] * nrhs + c0 +
+                       min(l16, g - 1)];
+        d4_t acc = {0.0, 0.0, 0.0, 0.0};
+        if (!first)
+            acc = bl_rows_times<double>(Ap + (int64_t)perm[min(i0 + l16, n - 1)] * n, xs, g, g, 0,
+                                        n);
 #pragma unroll
-        for (int c = 0; c < BL_MAXRHS; ++c) acc[c] = 0.0;
-        const int row = perm[min(i, n - 1)];       // unconditional; unused past n
-        if (i < n && !first) {
-            const double *ar = Ap + (int64_t)row * n;
-            // 8 independent row loads in flight per lane
-#pragma unroll 8
-            for (int j = l16; j < n; j += 16) {
-                const double a = ar[j];
-#pragma unroll
-                for (int c = 0; c < BL_MAXRHS; ++c)
-                    if (c < g) acc[c] = fma(a, xs[j * g + c], acc[c]);
+        for (int r = 0; r < 4; ++r) {
+            const int i = i0 + BlVec<double>::drow(lhi, r);
+            if (i < n && l16 < g) {
+                const double v = bv[r] - acc[r];
+                Y[i * g + l16] = (T)v;
+                rmax = fmax(rmax, fabs(v));
             }
         }
-        if (!first) {
-#pragma unroll
-            for (int c = 0; c < BL_MAXRHS; ++c)
-                if (c < g) {
-#pragma unroll
-                    for (int msk = 8; msk >= 1; msk >>= 1) acc[c] += __shfl_xor(acc[c], msk);
-                }
-        }
-        // the right-hand side row, loaded unconditionally (clamped column)
-        const double *br = Bp + (int64_t)row * nrhs + c0;
-        double bv[BL_MAXRHS];
-#pragma unroll
-        for (int c = 0; c < BL_MAXRHS; ++c) bv[c] = br[min(c, g - 1)];
-        if (i < n && l16 == 0) {
-#pragma unroll
-            for (int c = 0; c < BL_MAXRHS; ++c)
-                if (c < g) {
-                    const double r = bv[c] - acc[c];
-                    Y[i * g + c] = (T)r;
-                    rmax[c] = fmax(rmax[c], fabs(r));
-                }
-        }
     }
-#pragma unroll
-    for (int c = 0; c < BL_MAXRHS; ++c) {
-        const double v = bl_wave_max(rmax[c]);
-        if (lane == 0) L.red[wave * BL_MAXRHS + c] = v;
-    }
+    rmax = fmax(rmax, __shfl_xor(rmax, 16));
+    rmax = fmax(rmax, __shfl_xor(rmax, 32));
+    if (lane < BL_MAXRHS) L.red[wave * BL_MAXRHS + lane] = rmax;
     __syncthreads();
-#pragma unroll
-    for (int c = 0; c < BL_MAXRHS; ++c)
-        rn[c] = fmax(fmax(L.red[c], L.red[BL_MAXRHS + c]),
-                     fmax(L.red[2 * BL_MAXRHS + c], L.red[3 * BL_MAXRHS + c]));
+    if (tid < BL_MAXRHS)
+        L.rn[tid] = fmax(fmax(L.red[tid], L.red[BL_MAXRHS + tid]),
+                         fmax(L.red[2 * BL_MAXRHS + tid], L.red[3 * BL_MAXRHS + tid]));
     __syncthreads();
 }
 
-// x += Y (columns c0..c0+g-1); xn[c] = max |x_c| afterwards
+// x += Y (columns c0..c0+g-1); L.xn[c] = max |x_c| afterwards
 template <int MODE>
 __device__ void bl_update_x(int n, int nrhs, int c0, int g, double *Xp, BlLds<MODE> &L,
-                            bool first, double *xn)
+                            bool first)
 {
     typedef typename BlCfg<MODE>::T T;
     const T *Y = reinterpret_cast<const T *>(L.y);
@@ -628,10 +772,9 @@ __device__ void bl_update_x(int n, int nrhs, int c0, int g, double *Xp, BlLds<MO
         if (lane == 0) L.red[4 * BL_MAXRHS + wave * BL_MAXRHS + c] = v;
     }
     __syncthreads();
-#pragma unroll
-    for (int c = 0; c < BL_MAXRHS; ++c)
-        xn[c] = fmax(fmax(L.red[4 * BL_MAXRHS + c], L.red[5 * BL_MAXRHS + c]),
-                     fmax(L.red[6 * BL_MAXRHS + c], L.red[7 * BL_MAXRHS + c]));
+    if (tid < BL_MAXRHS)
+        L.xn[tid] = fmax(fmax(L.red[4 * BL_MAXRHS + tid], L.red[5 * BL_MAXRHS + tid]),
+                         fmax(L.red[6 * BL_MAXRHS + tid], L.red[7 * BL_MAXRHS + tid]));
     __syncthreads();
 }
 
@@ -652,25 +795,23 @@ __device__ void bl_refine(int n, int nrhs, const double *__restrict__ Ap,
     eta_out = 0.0;
     for (int c0 = 0; c0 < nrhs; c0 += gmax) {
         const int g = min(gmax, nrhs - c0);
-        double bn[BL_MAXRHS], xn[BL_MAXRHS], rn[BL_MAXRHS];
-#pragma unroll
-        for (int c = 0; c < BL_MAXRHS; ++c) { bn[c] = 0.0; xn[c] = 0.0; }
         double eta = 1.0, eta_prev = 1e300;
         int stalls = 0, it = 0;
         for (;; ++it) {
-            bl_residual<MODE>(n, nrhs, c0, g, it == 0, Ap, Bp, Xp, perm, L, rn);
+            bl_residual<MODE>(n, nrhs, c0, g, it == 0, Ap, Bp, Xp, perm, L);
             if (it == 0) {
-#pragma unroll
-                for (int c = 0; c < BL_MAXRHS; ++c) bn[c] = rn[c];
+                if (threadIdx.x < BL_MAXRHS) {
+                    L.bn[threadIdx.x] = L.rn[threadIdx.x];
+                    L.xn[threadIdx.x] = 0.0;
+                }
+                __syncthreads();
             }
             eta = 0.0;
-#pragma unroll
-            for (int c = 0; c < BL_MAXRHS; ++c)
-                if (c < g) {
-                    const double den = anorm * xn[c] + bn[c];
-                    const double e = den > 0.0 ? rn[c] / den : (rn[c] > 0.0 ? 1e300 : 0.0);
-                    eta = (e != e) ? 1e300 : fmax(eta, e);
-                }
+            for (int c = 0; c < g; ++c) {
+                const double den = anorm * L.xn[c] + L.bn[c], r = L.rn[c];
+                const double e = den > 0.0 ? r / den : (r > 0.0 ? 1e300 : 0.0);
+                eta = (e != e) ? 1e300 : fmax(eta, e);
+            }
             if (it > 0) {
                 if (eta <= tol) break;
                 if (MODE == LA_PREC_FP64) break;
@@ -682,8 +823,8 @@ __device__ void bl_refine(int n, int nrhs, const double *__restrict__ Ap,
                 }
             }
             eta_prev = eta;
-            bl_trsv_lu<T>(n, W, Y, g);
-            bl_update_x<MODE>(n, nrhs, c0, g, Xp, L, it == 0, xn);
+            bl_trsv_lu<T>(n, W, Y, g, L.stg);
+            bl_update_x<MODE>(n, nrhs, c0, g, Xp, L, it == 0);
         }
         iters = max(iters, it - 1);
         eta_out = fmax(eta_out, eta);
@@ -704,7 +845,8 @@ void k_lu_ir_batched(int count, const int32_t *__restrict__ order, const int32_t
     for (;;) {
         if (threadIdx.x == 0) L.prob = (int)atomicAdd(&queue[0], 1u);
         __syncthreads();
-        const int pi = L.prob;
+        // uniform: sizes and pointers of the problem stay in scalar registers
+        const int pi = __builtin_amdgcn_readfirstlane(L.prob);
         __syncthreads();
         if (pi >= count) break;
         const int prob = order[pi];
