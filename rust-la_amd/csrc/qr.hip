@@ -18,7 +18,8 @@
 //     (T upper triangular, T_jj = tau_j = -1/(a_j u_j), forward column-wise
 //     accumulation of Schreiber and Van Loan), applied to the trailing
 //     columns as A2 -= V (T^T (V^T A2)): V^T A2 (32 rows, long K) split over
-//     row chunks and summed in chunk order, the other two on MFMA.
+//     row chunks and summed in chunk order, T^T applied through its inverse
+//     (the Gram matrix of V), V times the rest by the GEMM.
 // get_q applies the blocks to the partial identity in reverse order
 // (Q = (I - V T V^T) Q), the least-squares solve applies them to B in
 // forward order and finishes with R x = (Q^T B)[0..n).
@@ -79,7 +80,7 @@ __device__ inline bool wait_tagged(const uint64_t *p, uint32_t tag, uint64_t &v,
 //      and its rows r >= gc get A[r][j] += f_j u_r (u_gc = u_c), A[gc][c] = u_c.
 // With want_vg the kernel also writes its rows of V (the Householder vectors,
 // as k_qr_make_v builds them) and its partial Gram matrix V_w^T V_w (on MFMA,
-// a fixed order) as chunk w of the partial products that k_qr_vtc_reduce
+// a fixed order) as chunk w of the partial products that k_qr_vtc
 // adds up, so the block's V^T V needs no pass over V.
 // A workgroup can publish column c + 2 into a buffer only after every
 // workgroup published column c + 1, which each did after reading column c,
@@ -400,63 +401,205 @@ void k_qr_apply(int m, double *__restrict__ A, int64_t lda, int c, int cend,
     }
 }
 
-// W = V^T C (nb x cols) for a tall V (rows x nb, ld nb) and C (rows x cols,
-// ld ldc): a product with a short output and a long K, split over row chunks
-// (blockIdx.y) whose partial products are summed by k_qr_vtc_reduce in chunk
-// order.  Thread t owns column (t & 127) of a 128-column tile and 16 of the
-// 32 rows of W; V is staged in LDS 64 rows at a time, zero past nb.
-constexpr int VT_COLS = 128, VT_SUB = 64, VT_MAXCHUNK = 16;
+// Partial products W = V^T C (nb x cols) of a tall V (rows x nb, ld nb) and C
+// (rows x cols, ld ldc), one per row chunk (blockIdx.y) and 32 columns
+// (blockIdx.x), for k_qr_tsolve to add up in chunk order; and the block's Gram
+// matrix G = V^T V in the last column of workgroups: the same product with
+// C = V, or (npg > 0) the sum of the panel kernel's npg partials.
+// A short output with a long K: both operands come straight from memory in
+// the MFMA layout (element i of a wave's step is V[r][i], C[r][i]: sixteen
+// consecutive doubles of four rows), sixteen rows at a time with the next
+// sixteen in flight; a wave takes every fourth sixteen of the chunk and the
+// four sums meet in LDS.  Bound by latency: 4096 x 32 against 992 columns
+// takes 8 us (52 with V staged in LDS and FP64 FMAs, two waves per column).
+constexpr int VT_COLS = 32, VT_MAXCHUNK = 16;
 __global__ __launch_bounds__(256)
-void k_qr_vtc_partial(int rows, int nb, int cols, int rch, const double *__restrict__ V,
-                      const double *__restrict__ C, int64_t ldc, double *__restrict__ P)
+void k_qr_vtc(int rows, int nb, int cols, int rch, const double *__restrict__ V,
+              const double *__restrict__ C, int64_t ldc, double *__restrict__ P, int npg,
+              double *__restrict__ PG, double *__restrict__ G)
 {
-    __shared__ double vs[VT_SUB][QR_NB];
-    const int t = threadIdx.x;
-    const int col = blockIdx.x * VT_COLS + (t & 127), jh = (t >> 7) * 16;
-    const int r0 = blockIdx.y * rch, r1 = min(rows, r0 + rch);
-    const bool okc = col < cols;
-    double acc[16];
+    __shared__ double red[4][QR_NB][VT_COLS + 1];
+    const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, lhi = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    int c0 = blockIdx.x * VT_COLS;
+    if (blockIdx.x == gridDim.x - 1) {
+        if (npg > 0) {
+            if (blockIdx.y == 0)
+                for (int e = t; e < nb * nb; e += 256) {
+                    double s = 0.0;
+                    for (int h0 = 0; h0 < npg; h0 += 16) {
+                        double v[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0.0;
-    for (int rs = r0; rs < r1; rs += VT_SUB) {
-        const int rn = min(VT_SUB, r1 - rs);
-        for (int e = t; e < VT_SUB * QR_NB; e += 256) {
-            const int rr = e / QR_NB, j = e - rr * QR_NB;
-            vs[rr][j] = (rr < rn && j < nb) ? V[(int64_t)(rs + rr) * nb + j] : 0.0;
-        }
-        __syncthreads();
-        const double *cp = C + (int64_t)rs * ldc + (okc ? col : 0);
-        // eight rows of C in flight per step (clamped loads, uniform guard)
-        for (int rr0 = 0; rr0 < rn; rr0 += 8) {
-            double cv[8];
+                        for (int h = 0; h < 16; ++h)
+                            v[h] = PG[(int64_t)min(h0 + h, npg - 1) * QR_NB * nb + e];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) cv[u] = cp[(int64_t)min(rr0 + u, rn - 1) * ldc];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (rr0 + u < rn) {
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) acc[j] = fma(vs[rr0 + u][jh + j], cv[u], acc[j]);
+                        for (int h = 0; h < 16; ++h)
+                            if (h0 + h < npg) s += v[h];
+                    }
+                    G[e] = s;
                 }
-            }
+            return;
         }
-        __syncthreads();
+        C = V;
+        ldc = nb;
+        cols = nb;
+        c0 = 0;
+        P = PG;
     }
-    if (okc)
+    const int r0 = blockIdx.y * rch, r1 = min(rows, r0 + rch);
+    // columns past nb and cols are clamped: their products are not stored
+    const int i0 = min(l16, nb - 1), i1 = min(16 + l16, nb - 1);
+    const int j0 = min(c0 + l16, cols - 1), j1 = min(c0 + 16 + l16, cols - 1);
+    d4_t acc[2][2];
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
-            if (jh + j < nb) P[((int64_t)blockIdx.y * QR_NB + jh + j) * cols + col] = acc[j];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = (d4_t){0.0, 0.0, 0.0, 0.0};
+    double a[4][2], b[4][2], an[4][2], bn[4][2];
+    auto load = [&](double (&x)[4][2], double (&y)[4][2], int rs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int r = min(rs + 4 * s + lhi, r1 - 1);
+            const double *v = V + (int64_t)r * nb, *c = C + (int64_t)r * ldc;
+            x[s][0] = v[i0];
+            x[s][1] = v[i1];
+            y[s][0] = c[j0];
+            y[s][1] = c[j1];
+        }
+    };
+    int rs = r0 + 16 * wave;
+    if (rs < r1) load(a, b, rs);
+    for (; rs < r1; rs += 64) {
+        if (rs + 64 < r1) load(an, bn, rs + 64);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (rs + 4 * s + lhi >= r1) {       // past the chunk: both operands zero
+                a[s][0] = a[s][1] = 0.0;
+                b[s][0] = b[s][1] = 0.0;
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][i], b[s][j], acc[i][j],
+                                                                     0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[s][i] = an[s][i];
+                b[s][i] = bn[s][i];
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                red[wave][16 * i + lhi + 4 * r][16 * j + l16] = acc[i][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int e = t + 256 * q, i = e >> 5, c = e & 31;
+        if (i < nb && c0 + c < cols)
+            P[((int64_t)blockIdx.y * QR_NB + i) * cols + c0 + c] =
+                (red[0][i][c] + red[1][i][c]) + (red[2][i][c] + red[3][i][c]);
+    }
 }
 
+// W2 = op(T) W for W = the sum of nch partials P (nb x cols) and the T of
+// I - V T V^T = H_0 ... H_nb-1.  T itself is never formed: with G = V^T V and
+// tau_j = -1/(a_j u_j) (0 for a skipped column) its inverse is upper
+// triangular, 1/tau_j on the diagonal and G above it, so
+//   op = T^T:  x_j = tau_j (w_j - sum_{i<j} G_ij x_i),  j ascending
+//   op = T  :  x_j = tau_j (w_j - sum_{i>j} G_ji x_i),  j descending,
+// one column per thread.  G comes as npg partials.
 __global__ __launch_bounds__(256)
-void k_qr_vtc_reduce(int nchunks, int nb, int cols, const double *__restrict__ P,
-                     double *__restrict__ W)
+void k_qr_tsolve(int nb, int cols, int nch, const double *__restrict__ P, int npg,
+                 const double *__restrict__ PG, const double *__restrict__ rd,
+                 const double *__restrict__ diagu, int64_t ldu, int trans,
+                 double *__restrict__ W2)
 {
-    const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;
-    if (e >= (int64_t)nb * cols) return;
-    const int j = (int)(e / cols), col = (int)(e - (int64_t)j * cols);
-    double s = 0.0;
-    for (int ch = 0; ch < nchunks; ++ch) s += P[((int64_t)ch * QR_NB + j) * cols + col];
-    W[(int64_t)j * cols + col] = s;
+    __shared__ double G[QR_NB][QR_NB + 2], W[QR_NB][VT_COLS + 1], tau[QR_NB];
+    const int t = threadIdx.x, c0 = blockIdx.x * VT_COLS;
+    double w[4], g[4];
+    // v += the partials' elements, four partials' loads in flight at a time
+    auto sum = [&](double (&v)[4], const double *src, int64_t ld, int64_t stride, int c,
+                   int n) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = 0.0;
+        for (int h0 = 0; h0 < n; h0 += 4) {
+            double x[4][4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    x[h][q] = src[min(h0 + h, n - 1) * stride + min((t >> 5) + 8 * q, nb - 1) * ld + c];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                if (h0 + h < n)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] += x[h][q];
+        }
+    };
+    sum(g, PG, nb, (int64_t)QR_NB * nb, min(t & 31, nb - 1), npg);
+    sum(w, P, cols, (int64_t)QR_NB * cols, min(c0 + (t & 31), cols - 1), nch);
+    if (t < QR_NB) {
+        const int jc = min(t, nb - 1);
+        const double a = rd[jc], u = diagu[(int64_t)jc * ldu + jc];
+        tau[t] = (t < nb && a != 0.0) ? -1.0 / (a * u) : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int e = t + 256 * q, i = e >> 5, c = e & 31;
+        W[i][c] = i < nb ? w[q] : 0.0;
+        G[i][c] = i < nb && c < nb ? g[q] : 0.0;
+    }
+    __syncthreads();
+    // one column per thread, eight rows at a time: finished blocks come back
+    // from LDS.  Rolled over the blocks, because straight-line code that runs
+    // once waits for its instructions (all 32 rows unrolled: 14 us).  Rows
+    // past nb are zero.
+    if (t < VT_COLS) {
+        constexpr int B = 8;
+        for (int bi = 0; bi < QR_NB / B; ++bi) {
+            const int b0 = B * (trans ? bi : QR_NB / B - 1 - bi);
+            double x[B];
+#pragma unroll
+            for (int i = 0; i < B; ++i) x[i] = W[b0 + i][t];
+            for (int ki = 0; ki < bi; ++ki) {
+                const int k0 = B * (trans ? ki : QR_NB / B - 1 - ki);
+#pragma unroll
+                for (int k = 0; k < B; ++k) {
+                    const double y = W[k0 + k][t];
+#pragma unroll
+                    for (int i = 0; i < B; ++i) x[i] = fma(-G[k0 + k][b0 + i], y, x[i]);
+                }
+            }
+            if (trans) {
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    x[j] *= tau[b0 + j];
+#pragma unroll
+                    for (int i = j + 1; i < B; ++i) x[i] = fma(-G[b0 + j][b0 + i], x[j], x[i]);
+                }
+            } else {
+#pragma unroll
+                for (int j = B - 1; j >= 0; --j) {
+                    x[j] *= tau[b0 + j];
+#pragma unroll
+                    for (int i = 0; i < j; ++i) x[i] = fma(-G[b0 + j][b0 + i], x[j], x[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < B; ++i) {
+                W[b0 + i][t] = x[i];
+                if (b0 + i < nb && c0 + t < cols) W2[(int64_t)(b0 + i) * cols + c0 + t] = x[i];
+            }
+        }
+    }
 }
 
 // V (rows x nb, ld nb) of the panel's Householder vectors: column j is zero
@@ -472,62 +615,6 @@ void k_qr_make_v(int rows, int nb, const double *__restrict__ A, int64_t lda,
     double v = 0.0;
     if (r >= j && rd[j] != 0.0) v = A[(int64_t)r * lda + j];
     V[(int64_t)r * nb + j] = v;
-}
-
-// T (nb x nb, upper) of I - V T V^T = H_0 ... H_nb-1 from the Gram matrix
-// G = V^T V: T_jj = tau_j, T[0:j, j] = -tau_j T[0:j, 0:j] G[0:j, j]
-// (tau_j = -1/(a_j u_j), 0 for a skipped column).  One workgroup; also
-// writes Tt = T^T.
-__global__ __launch_bounds__(64)
-void k_qr_larft(int nb, const double *__restrict__ G, const double *__restrict__ rd,
-                const double *__restrict__ diagu, int64_t ldu, double *__restrict__ T,
-                double *__restrict__ Tt)
-{
-    __shared__ double sT[QR_NB][QR_NB + 1], sG[QR_NB][QR_NB + 1];
-    __shared__ double stau[QR_NB];
-    const int t = threadIdx.x;
-    // G, rdiag and the diagonal of u staged in LDS first: the recurrence
-    // below then issues no global load
-    for (int e = t; e < QR_NB * QR_NB; e += 64) {
-        const int i = e / QR_NB, j = e % QR_NB;
-        sT[i][j] = 0.0;
-        const double g = G[min(i, nb - 1) * nb + min(j, nb - 1)];
-        sG[i][j] = (i < nb && j < nb) ? g : 0.0;
-    }
-    if (t < QR_NB) {
-        const int jc = min(t, nb - 1);
-        const double a = rd[jc], u = diagu[(int64_t)jc * ldu + jc];
-        stau[t] = (t < nb && a != 0.0) ? -1.0 / (a * u) : 0.0;
-    }
-    __syncthreads();
-    // thread t < 32 keeps row t of T in registers; per column j it forms
-    // w_t = sum_{q = t}^{j-1} T[t][q] G[q][j] (q ascending, as the textbook
-    // recurrence) from LDS broadcasts of G's column, with no barrier
-    double tr[QR_NB];
-#pragma unroll
-    for (int q = 0; q < QR_NB; ++q) tr[q] = 0.0;
-#pragma unroll
-    for (int j = 0; j < QR_NB; ++j) {
-        if (j < nb) {
-            double s = 0.0;
-#pragma unroll
-            for (int q = 0; q < j; ++q) {
-                const double g = sG[q][j];
-                if (q >= t) s += tr[q] * g;
-            }
-            if (t < j) tr[j] = -stau[j] * s;
-            else if (t == j) tr[j] = stau[j];
-        }
-    }
-    if (t < QR_NB)
-#pragma unroll
-        for (int q = 0; q < QR_NB; ++q) sT[t][q] = tr[q];
-    __syncthreads();
-    for (int e = t; e < nb * nb; e += 64) {
-        const int i = e / nb, j = e % nb;
-        T[e] = sT[i][j];
-        Tt[e] = sT[j][i];
-    }
 }
 
 // Q = partial identity (ones at (i, i) for i < dc), m x m, ld ldq.
@@ -568,68 +655,52 @@ void k_qr_copy(int rows, int cols, const double *__restrict__ B, int64_t ldb,
 
 namespace {
 
-// Workspace of one QR call.
+// Workspace of one QR call.  pool holds the partial Gram matrices of a block
+// (a chunk is QR_NB x nb), then the partial products of V^T C.
 struct QrWs {
-    double *V, *G, *T, *Tt, *W, *W2, *npart, *dpart, *scal, *P;
+    double *V, *G, *W2, *npart, *dpart, *scal, *pool;
+    size_t pool_bytes;
     uint64_t *slots;
 };
+constexpr size_t QR_G_BYTES = (size_t)QR_NB * QR_NB * 8;
 
 int qr_ws(la_ctx *ctx, int64_t m, int64_t n, int64_t wcols, QrWs &w)
 {
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const int64_t dc = std::min(m, n);
-    const size_t bv = al((size_t)m * QR_NB * 8), bg = al((size_t)QR_NB * QR_NB * 8),
-                 bw = al((size_t)QR_NB * std::max<int64_t>(wcols, 1) * 8),
+    const int64_t dc = std::min(m, n), wc = std::max<int64_t>(wcols, 1);
+    const size_t bv = al((size_t)m * QR_NB * 8), bw = al((size_t)QR_NB * wc * 8),
                  bp = al((size_t)QR_PARTS * 8), bd = al((size_t)QR_PARTS * QR_NB * 8),
                  bs = al((size_t)2 * std::max<int64_t>(dc, 1) * 8),
-                 bpk = al(std::max((size_t)VT_MAXCHUNK * QR_NB * std::max<int64_t>(std::max<int64_t>(wcols, 1), QR_NB) * 8,
-                                   (size_t)QRP_MAXP * QR_NB * QR_NB * 8));
-    const size_t bsl = al((size_t)2 * QRP_MAXP * QRP_SW * 8);
-    void *base = nullptr;
-    int st = ws_get(ctx, WS_QR, bv + 3 * bg + 2 * bw + bp + bd + bs + bpk + bsl, &base);
-    if (st) return st;
+                 bsl = al((size_t)2 * QRP_MAXP * QRP_SW * 8);
+    const size_t fixed = bv + QR_G_BYTES + bw + bp + bd + bs + bsl;
+    // room for every partial; under a workspace limit the least that holds a
+    // panel's Gram partials beside one chunk of products (fewer, longer
+    // chunks: qr_chunks)
+    const size_t full = (size_t)QRP_MAXP * QR_G_BYTES + (size_t)VT_MAXCHUNK * bw;
+    const size_t least = std::max((size_t)VT_MAXCHUNK * bw, (size_t)QRP_MAXP * QR_G_BYTES) + bw +
+                         2 * QR_G_BYTES;
+    w.pool_bytes = std::max(full, least);
+    void *base = ws_try(ctx, WS_QR, fixed + w.pool_bytes);
+    if (!base) {
+        w.pool_bytes = least;
+        int st = ws_get(ctx, WS_QR, fixed + least, &base);
+        if (st) return st;
+    }
     char *p = (char *)base;
     w.V = (double *)p; p += bv;
-    w.G = (double *)p; p += bg;
-    w.T = (double *)p; p += bg;
-    w.Tt = (double *)p; p += bg;
-    w.W = (double *)p; p += bw;
+    w.G = (double *)p; p += QR_G_BYTES;
     w.W2 = (double *)p; p += bw;
     w.npart = (double *)p; p += bp;
     w.dpart = (double *)p; p += bd;
     w.scal = (double *)p; p += bs;
-    w.P = (double *)p; p += bpk;
+    w.pool = (double *)p; p += w.pool_bytes;
     w.slots = (uint64_t *)p;
     return LA_OK;
 }
 
 int grid_rows(int64_t rows) { return (int)std::min<int64_t>(QR_PARTS, std::max<int64_t>(1, ceil_div(rows, 256))); }
 
-// W (nb x cols, ld cols) = V^T C, split over at most VT_MAXCHUNK row chunks
-int qr_vtc(la_ctx *ctx, int64_t rows, int nb, int64_t cols, const double *C, int64_t ldc,
-           double *W, QrWs &w)
-{
-    const int64_t rch = std::max<int64_t>(VT_SUB, ceil_div(ceil_div(rows, VT_MAXCHUNK), VT_SUB) * VT_SUB);
-    const int nch = (int)ceil_div(rows, rch);
-    hipLaunchKernelGGL(k_qr_vtc_partial, dim3((unsigned)ceil_div(cols, VT_COLS), (unsigned)nch),
-                       dim3(256), 0, ctx->stream, (int)rows, nb, (int)cols, (int)rch,
-                       (const double *)w.V, C, ldc, w.P);
-    hipLaunchKernelGGL(k_qr_vtc_reduce, dim3((unsigned)ceil_div(nb * cols, 256)), dim3(256), 0,
-                       ctx->stream, nch, nb, (int)cols, (const double *)w.P, W);
-    LA_HIP_CHECK(ctx, hipGetLastError());
-    return LA_OK;
-}
-
-// T of a panel from its G = V^T V (in w.G); diagu: the panel's diagonal block.
-int qr_larft(la_ctx *ctx, int nb, const double *rd, const double *diagu, int64_t ldu, QrWs &w)
-{
-    hipLaunchKernelGGL(k_qr_larft, dim3(1), dim3(64), 0, ctx->stream, nb, (const double *)w.G,
-                       rd, diagu, ldu, w.T, w.Tt);
-    LA_HIP_CHECK(ctx, hipGetLastError());
-    return LA_OK;
-}
-
-// V and T of the panel at column k0 (width nb) of the packed factor.
+// V of the panel at column k0 (width nb) of the packed factor.
 int qr_block(la_ctx *ctx, int64_t m, const double *QR, int64_t ldq, const double *rdiag,
              int64_t k0, int nb, QrWs &w)
 {
@@ -637,22 +708,33 @@ int qr_block(la_ctx *ctx, int64_t m, const double *QR, int64_t ldq, const double
     hipLaunchKernelGGL(k_qr_make_v, dim3((unsigned)ceil_div(rows * nb, 256)), dim3(256), 0,
                        ctx->stream, (int)rows, nb, QR + k0 * ldq + k0, ldq, rdiag + k0, w.V);
     LA_HIP_CHECK(ctx, hipGetLastError());
-    int st = qr_vtc(ctx, rows, nb, nb, w.V, nb, w.G, w);
-    if (st) return st;
-    return qr_larft(ctx, nb, rdiag + k0, QR + k0 * ldq + k0, ldq, w);
+    return LA_OK;
 }
 
 // C (rows x cols, ld ldc, the rows k0.. of the operand) <- (I - V op(T) V^T) C
-// with op(T) = T^T (trans) or T.
+// with op(T) = T^T (trans) or T, for the block's V in w.V, its rdiag entries
+// and its diagonal block (of which the diagonal, u, is read).  npg: partials
+// of V^T V that the panel kernel left at the start of w.pool, or 0.
 int qr_apply_block(la_ctx *ctx, int64_t rows, int nb, int64_t cols, double *C, int64_t ldc,
-                   bool trans, QrWs &w)
+                   bool trans, const double *rd, const double *diagu, int64_t ldu, int npg,
+                   QrWs &w)
 {
     if (cols <= 0) return LA_OK;
-    int st = qr_vtc(ctx, rows, nb, cols, C, ldc, w.W, w);
-    if (st) return st;
-    st = gemm_rm<double>(ctx, nb, cols, nb, 1.0, trans ? w.Tt : w.T, nb, w.W, cols, 0.0, w.W2,
-                         cols, false, false);
-    if (st) return st;
+    // row chunks: multiples of 64 rows, as many as fill the device and as
+    // their partials fit
+    const size_t gbytes = (size_t)(npg > 0 ? npg : VT_MAXCHUNK) * QR_G_BYTES;
+    const int64_t fit = (int64_t)((w.pool_bytes - gbytes) / ((size_t)QR_NB * cols * 8));
+    const int64_t maxch = std::max<int64_t>(1, std::min<int64_t>(VT_MAXCHUNK, fit));
+    const int64_t rch = ceil_div(ceil_div(rows, maxch), 64) * 64;
+    const int nch = (int)ceil_div(rows, rch);
+    double *PG = w.pool, *P = w.pool + gbytes / 8;
+    hipLaunchKernelGGL(k_qr_vtc, dim3((unsigned)ceil_div(cols, VT_COLS) + 1, (unsigned)nch),
+                       dim3(256), 0, ctx->stream, (int)rows, nb, (int)cols, (int)rch,
+                       (const double *)w.V, (const double *)C, ldc, P, npg, PG, w.G);
+    hipLaunchKernelGGL(k_qr_tsolve, dim3((unsigned)ceil_div(cols, VT_COLS)), dim3(256), 0,
+                       ctx->stream, nb, (int)cols, nch, (const double *)P, npg > 0 ? 1 : nch,
+                       (const double *)(npg > 0 ? w.G : PG), rd, diagu, ldu, trans ? 1 : 0, w.W2);
+    LA_HIP_CHECK(ctx, hipGetLastError());
     return gemm_rm<double>(ctx, rows, cols, nb, -1.0, w.V, nb, w.W2, cols, 1.0, C, ldc, false,
                            false);
 }
@@ -703,21 +785,15 @@ int geqrf_device(la_ctx *ctx, int64_t m, int64_t n, double *A, int64_t lda, doub
             uint64_t tk = ticks;
             int want = cend < n ? 1 : 0;
             void *args[] = {&mi, &A, &lda, &k0i, (void *)&nb, &rdiag, &w.slots, &stp, &tk,
-                            &w.V, &w.P, &want};
+                            &w.V, &w.pool, &want};
             // an ordinary launch: at most 128 workgroups of one per CU are
             // co-resident on the full device, every wait is bounded, and the
             // cooperative-launch API would tie the device to this process
             // (another process's cooperative launch then fails)
             LA_HIP_CHECK(ctx, hipLaunchKernel(fn, dim3(Pq), dim3(256), args, shmem, ctx->stream));
             if (want) {
-                // the block's V^T V from the panel's per-workgroup partials, then T
-                hipLaunchKernelGGL(k_qr_vtc_reduce, dim3((unsigned)ceil_div(nb * nb, 256)),
-                                   dim3(256), 0, ctx->stream, Pq, nb, nb, (const double *)w.P,
-                                   w.G);
-                LA_HIP_CHECK(ctx, hipGetLastError());
-                if ((st = qr_larft(ctx, nb, rdiag + k0, A + k0 * lda + k0, lda, w))) return st;
                 if ((st = qr_apply_block(ctx, m - k0, nb, n - cend, A + k0 * lda + cend, lda,
-                                         true, w)))
+                                         true, rdiag + k0, A + k0 * lda + k0, lda, Pq, w)))
                     return st;
             }
             continue;
@@ -744,7 +820,8 @@ int geqrf_device(la_ctx *ctx, int64_t m, int64_t n, double *A, int64_t lda, doub
         // the block's reflections on the trailing columns
         if (cend < n) {
             if ((st = qr_block(ctx, m, A, lda, rdiag, k0, nb, w))) return st;
-            if ((st = qr_apply_block(ctx, m - k0, nb, n - cend, A + k0 * lda + cend, lda, true, w)))
+            if ((st = qr_apply_block(ctx, m - k0, nb, n - cend, A + k0 * lda + cend, lda, true,
+                                     rdiag + k0, A + k0 * lda + k0, lda, 0, w)))
                 return st;
         }
     }
@@ -766,7 +843,9 @@ int qr_q_device(la_ctx *ctx, int64_t m, int64_t n, const double *QR, int64_t ldq
     for (int64_t k0 = last; k0 >= 0; k0 -= QR_NB) {
         const int nb = (int)std::min<int64_t>(QR_NB, dc - k0);
         if ((st = qr_block(ctx, m, QR, ldqr, rdiag, k0, nb, w))) return st;
-        if ((st = qr_apply_block(ctx, m - k0, nb, m, Q + k0 * ldq, ldq, false, w))) return st;
+        if ((st = qr_apply_block(ctx, m - k0, nb, m, Q + k0 * ldq, ldq, false, rdiag + k0,
+                                 QR + k0 * ldqr + k0, ldqr, 0, w)))
+            return st;
     }
     return LA_OK;
 }
@@ -783,7 +862,9 @@ int qr_solve_device(la_ctx *ctx, int64_t m, int64_t n, const double *QR, int64_t
     for (int64_t k0 = 0; k0 < n; k0 += QR_NB) {
         const int nb = (int)std::min<int64_t>(QR_NB, n - k0);
         if ((st = qr_block(ctx, m, QR, ldqr, rdiag, k0, nb, w))) return st;
-        if ((st = qr_apply_block(ctx, m - k0, nb, nx, Y + k0 * ldy, ldy, true, w))) return st;
+        if ((st = qr_apply_block(ctx, m - k0, nb, nx, Y + k0 * ldy, ldy, true, rdiag + k0,
+                                 QR + k0 * ldqr + k0, ldqr, 0, w)))
+            return st;
     }
     // R x = y[0..n): R with rdiag on its diagonal, solved as an upper factor
     hipLaunchKernelGGL(k_qr_make_r, dim3((unsigned)ceil_div(n * n, 256)), dim3(256), 0,
