@@ -608,20 +608,6 @@ void k_getrf_panel(T *A, int64_t lda, int M, int NB, int R, int kglob, int64_t *
     if (w == 0 && wave == 1) invert_unit_lower_wave<T>(blk, LDB, NB, linv);
 }
 
-// L11^-1 of the block's 64 x 64 diagonal triangles (one workgroup each), for
-// U12, from the factored block (Lblk, nbo columns).
-template <typename T>
-__global__ __launch_bounds__(256)
-void k_block_linv(const T *Lblk, int64_t lda, int nbo, T *linv)
-{
-    __shared__ T L[NB_IN * (NB_IN + 1)];
-    const int b = blockIdx.x, nb = min(NB_IN, nbo - b * NB_IN);
-    stage_block(L, NB_IN + 1, Lblk + (int64_t)b * NB_IN * (lda + 1), lda, nb, nb);
-    __syncthreads();
-    if (threadIdx.x < 64)
-        invert_unit_lower_wave<T>(L, NB_IN + 1, nb, linv + (size_t)b * NB_IN * NB_IN);
-}
-
 // ------------------------------------------------------ single-WG panel
 // Used when the whole M x NB panel fits one workgroup's LDS.  Column j is
 // formed LEFT-looking in exactly the reference's operation order
@@ -889,112 +875,6 @@ void k_trsm_unit_lower(const T *Linv, int nb, T *B, int64_t ldb, int ncols)
     }
 }
 
-// ------------------------------------------------------ block U12 = L11^-1 A12
-// U12 for an outer block of nbo <= NB_OUT rows in one pass.  Each workgroup
-// keeps CW columns of A12 (nbo x CW) in LDS and runs the block forward
-// substitution: for each 64-row panel b, X_b <- Linv_b X_b (the panel
-// kernel's inverse, unit diagonal implied; same operation order as
-// k_trsm_unit_lower), then X_r -= L_rb X_b for every panel r below it, with
-// L_rb read from the factored block (Lblk = A + K0 * lda + K0).  Replaces
-// per block four TRSM and three GEMM launches.  CW = 8 (FP32) or 16 (FP64).
-template <typename T, int CW>
-__global__ __launch_bounds__(256)
-void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ linv, int nbo,
-                 T *B, int64_t ldb, int ncols)
-{
-    constexpr int RQ = 256 / CW;            // row groups
-    constexpr int KR = 64 / RQ;             // rows per thread per 64-row panel
-    constexpr int XS = CW + 1, LS = 64 + 1;
-    extern __shared__ __align__(16) unsigned char u12_smem[];
-    T *X = reinterpret_cast<T *>(u12_smem);           // NB_OUT x XS
-    T *Ls = X + NB_OUT * XS;                          // 2 x 64 x LS
-    const int tid = threadIdx.x, cl = tid % CW, rq = tid / CW;
-    const int c0 = blockIdx.x * CW;
-    const int col = min(c0 + cl, ncols - 1);
-    const int nb = (nbo + 63) / 64;
-    // stages in order: for each panel b, its inverse (diagonal stage), then
-    // L_rb for r = b+1 .. nb-1; stage s + 1's 64 x 64 operand is loaded into
-    // registers while stage s computes, so the loads overlap the FMAs
-    const int nstage = nb + nb * (nb - 1) / 2;
-    auto stage_br = [&](int st, int &b, int &r) {
-        b = 0;
-        while (st >= nb - b) { st -= nb - b; ++b; }
-        r = b + st;                         // r == b: diagonal stage
-    };
-    T pre[16];
-    auto load_stage = [&](int st) {
-        int b, r;
-        stage_br(st, b, r);
-        const int nbb = min(64, nbo - 64 * b), nbr = min(64, nbo - 64 * r);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int e = tid + 256 * k, i = e >> 6, t = e & 63;
-            pre[k] = r == b ? linv[(size_t)b * NB_IN * NB_IN + min(i, nbb - 1) * NB_IN + min(t, nbb - 1)]
-                            : Lblk[(int64_t)(64 * r + min(i, nbr - 1)) * lda + 64 * b + min(t, nbb - 1)];
-        }
-    };
-    auto store_stage = [&](int st, T *dst) {
-        int b, r;
-        stage_br(st, b, r);
-        const int nbb = min(64, nbo - 64 * b), nbr = min(64, nbo - 64 * r);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int e = tid + 256 * k, i = e >> 6, t = e & 63;
-            const bool in = r == b ? (i < nbb && t < nbb && t != i) : (i < nbr && t < nbb);
-            dst[i * LS + t] = in ? pre[k] : T(0);
-        }
-    };
-    load_stage(0);
-    if constexpr (sizeof(T) == 8) {
-        // FP64: this thread's NB_OUT / RQ rows of the block, all loads in
-        // flight before the first store (measured: 1% off the FP64 LU; the
-        // same change slows the FP32 instance, which keeps the loop)
-        constexpr int NX = NB_OUT / RQ;
-        T xv[NX];
-#pragma unroll
-        for (int k = 0; k < NX; ++k) xv[k] = B[(int64_t)min(rq + RQ * k, nbo - 1) * ldb + col];
-#pragma unroll
-        for (int k = 0; k < NX; ++k) {
-            const int i = rq + RQ * k;
-            X[i * XS + cl] = i < nbo ? xv[k] : T(0);
-        }
-    } else {
-        for (int i = rq; i < NB_OUT; i += RQ) {
-            const T v = B[(int64_t)min(i, nbo - 1) * ldb + col];
-            X[i * XS + cl] = i < nbo ? v : T(0);
-        }
-    }
-    store_stage(0, Ls);
-    for (int st = 0; st < nstage; ++st) {
-        T *cur = Ls + (st & 1) * 64 * LS;
-        __syncthreads();                    // stage operand and X rows in place
-        if (st + 1 < nstage) load_stage(st + 1);
-        int b, r;
-        stage_br(st, b, r);
-        T acc[KR];
-#pragma unroll
-        for (int k = 0; k < KR; ++k) acc[k] = r == b ? X[(64 * b + rq + RQ * k) * XS + cl] : T(0);
-#pragma unroll 4
-        for (int t = 0; t < 64; ++t) {
-            const T xb = X[(64 * b + t) * XS + cl];
-#pragma unroll
-            for (int k = 0; k < KR; ++k) acc[k] += cur[(rq + RQ * k) * LS + t] * xb;
-        }
-        if (r == b) {
-            __syncthreads();                // every read of X_b is done
-#pragma unroll
-            for (int k = 0; k < KR; ++k) X[(64 * b + rq + RQ * k) * XS + cl] = acc[k];
-        } else {
-#pragma unroll
-            for (int k = 0; k < KR; ++k) X[(64 * r + rq + RQ * k) * XS + cl] -= acc[k];
-        }
-        if (st + 1 < nstage) store_stage(st + 1, Ls + ((st + 1) & 1) * 64 * LS);
-    }
-    __syncthreads();
-    if (c0 + cl < ncols)
-        for (int i = rq; i < nbo; i += RQ) B[(int64_t)i * ldb + c0 + cl] = X[i * XS + cl];
-}
-
 // sign = parity of the number of real swaps in ipiv (lu.rs:140-152 flips the
 // sign once per p != j).
 __global__ __launch_bounds__(256)
@@ -1177,37 +1057,6 @@ static int launch_trsm(la_ctx *ctx, const T *Linv, int nb, T *B, int64_t ldb, in
     return LA_OK;
 }
 
-template <typename T, int CW>
-static int launch_u12_cw(la_ctx *ctx, const T *Lblk, int64_t lda, const T *linv, int nbo,
-                         T *B, int64_t ldb, int64_t ncols)
-{
-    const void *fn = (const void *)k_u12_block<T, CW>;
-    const size_t shmem = ((size_t)NB_OUT * (CW + 1) + 2 * 64 * 65) * sizeof(T);
-    static size_t lm = 0;
-    if (!lm) lm = allow_dynamic_lds(fn);
-    if (shmem > lm) return set_error(ctx, LA_ERR_ARG, "getrf: U12 block exceeds LDS");
-    ProfScope ps(ctx, LA_K_TRSM, (double)nbo * nbo * ncols,
-                 (double)sizeof(T) * (2.0 * nbo * ncols + (double)nbo * nbo));
-    hipLaunchKernelGGL((k_u12_block<T, CW>), dim3((unsigned)ceil_div(ncols, (int64_t)CW)),
-                       dim3(256), shmem, ctx->stream, Lblk, lda, linv, nbo, B, ldb, (int)ncols);
-    LA_HIP_CHECK(ctx, hipGetLastError());
-    return LA_OK;
-}
-
-template <typename T>
-static int launch_u12_block(la_ctx *ctx, const T *Lblk, int64_t lda, const T *linv, int nbo,
-                            T *B, int64_t ldb, int64_t ncols)
-{
-    // columns per workgroup, measured at n = 16384 with look-ahead (FP32-IR
-    // 92.0 / 92.4 / 93.2 ms, FP64 LU 119.0 / 114.9 / 116.8 ms for 8 / 16 / 32):
-    // narrow workgroups shorten the U12 of the next block's 256 columns,
-    // which the next panel waits for
-    if constexpr (sizeof(T) == 4)
-        return launch_u12_cw<T, 8>(ctx, Lblk, lda, linv, nbo, B, ldb, ncols);
-    else
-        return launch_u12_cw<T, 16>(ctx, Lblk, lda, linv, nbo, B, ldb, ncols);
-}
-
 // Trailing updates: native MFMA for T, or FP32 data with BF16/FP16-rounded
 // operands on the low-precision MFMA (upd_prec = LA_PREC_BF16 / LA_PREC_FP16).
 template <typename T>
@@ -1242,7 +1091,7 @@ constexpr size_t NOALLOC_PUB_OFF = NOALLOC_PANEL_BYTES + NOALLOC_MAX_K * sizeof(
 constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PUB_OFF + BLK_PUB_BYTES;
 
 // The block (M rows, nbo columns at Ablk) in one launch, then its L11^-1
-// blocks.  One workgroup per CU at most (the tall layouts fill a CU's
+// blocks (linvs: null when no column right of the block needs them).  One workgroup per CU at most (the tall layouts fill a CU's
 // registers), nbo / cw of them, all resident at once on the whole device or
 // on the panel stream's CUs (checked by the caller).
 template <typename T>
@@ -1256,10 +1105,7 @@ static int launch_block(la_ctx *ctx, const BlockCfg &cfg, T *Ablk, int64_t lda, 
         LA_HIP_CHECK(ctx, hipLaunchKernel(cfg.fn, dim3((unsigned)ceil_div(nbo, cfg.cw)),
                                           dim3(cfg.nt), args, cfg.lds, ctx->stream));
     }
-    hipLaunchKernelGGL(k_block_linv<T>, dim3((unsigned)ceil_div(nbo, NB_IN)), dim3(256), 0,
-                       ctx->stream, (const T *)Ablk, lda, nbo, linvs);
-    LA_HIP_CHECK(ctx, hipGetLastError());
-    return LA_OK;
+    return linvs ? launch_block_linv<T>(ctx, Ablk, lda, nbo, linvs) : LA_OK;
 }
 
 template <typename T>
@@ -1513,7 +1359,7 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
         if (const BlockCfg *bc = block_for(K0)) {
             if ((st = launch_block<T>(ctx, *bc, A + K0 * lda + K0, lda, (int)(m - K0), (int)nbo,
                                       (int)K0, d_ipiv, pub, pv, pw.swapmap, d_status, ticks,
-                                      linv_ring)))
+                                      K0 + nbo < n ? linv_ring : (T *)nullptr)))
                 return st;
             if ((st = launch_block_moves<T>(ctx, A, lda, n, K0, K0 + nbo, pw.swapmap, d_perm)))
                 return st;
