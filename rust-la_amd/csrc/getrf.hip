@@ -1105,7 +1105,7 @@ static int launch_block(la_ctx *ctx, const BlockCfg &cfg, T *Ablk, int64_t lda, 
         LA_HIP_CHECK(ctx, hipLaunchKernel(cfg.fn, dim3((unsigned)ceil_div(nbo, cfg.cw)),
                                           dim3(cfg.nt), args, cfg.lds, ctx->stream));
     }
-    return linvs ? launch_block_linv<T>(ctx, Ablk, lda, nbo, linvs) : LA_OK;
+    return linvs ? launch_block_inv<T>(ctx, false, Ablk, lda, nbo, linvs) : LA_OK;
 }
 
 template <typename T>
@@ -1330,8 +1330,8 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
                          const T *linvs) -> int {
         if (ncol <= 0) return LA_OK;
         if (upd_prec != LA_PREC_BF16 && upd_prec != LA_PREC_FP16)
-            return launch_u12_block<T>(ctx, A + K0 * lda + K0, lda, linvs, (int)nbo,
-                                       A + K0 * lda + c0, lda, ncol);
+            return launch_trsm_block<T>(ctx, false, A + K0 * lda + K0, lda, linvs, (int)nbo,
+                                        A + K0 * lda + c0, lda, ncol);
         for (int64_t kb = K0; kb < K0 + nbo; kb += NB_IN) {
             const int nbi = (int)std::min<int64_t>(NB_IN, K0 + nbo - kb);
             const T *linv_kb = linvs + (size_t)((kb - K0) / NB_IN) * NB_IN * NB_IN;

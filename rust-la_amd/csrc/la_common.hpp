@@ -193,13 +193,13 @@ int trsv_blocked(la_ctx *ctx, char uplo, bool trans, bool unit, int64_t n,
                  const TF *Tm, int64_t ldt, int64_t nrhs, double *X, int64_t ldx);
 int gather_rows(la_ctx *ctx, int64_t m, int64_t nx, const uint64_t *d_piv, const double *B,
                 int64_t ldb, double *X, int64_t ldx);
-// X <- T^-1 X for many right-hand sides: blocked TRSM on the FP64 MFMA GEMM
+// X <- T^-1 X for several right-hand sides: blocked TRSM on the FP64 MFMA GEMM
 // with inverted 64 x 64 diagonal blocks ('L' unit lower / 'U' upper of a
 // packed LU)
 int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ldt, int64_t nrhs,
                  double *X, int64_t ldx);
 // right-hand-side counts from which the LU solves use trsm_blocked
-constexpr int64_t TRSM_MIN_RHS = 17, TRSM_MIN_N = 65;
+constexpr int64_t TRSM_MIN_RHS = 2, TRSM_MIN_N = 65;
 
 int potrf_blocked(la_ctx *ctx, int64_t n, double *A, int64_t lda, int32_t *d_status);
 

@@ -81,12 +81,13 @@ template <typename T> const BlockCfg *block_cfg(int64_t M, int num_cus);
 // Published multipliers of a block: NB_OUT columns of the tallest layout.
 constexpr size_t BLK_PUB_BYTES = (size_t)NB_OUT * 8192 * sizeof(double);
 
-// Inverses of a factored block's 64 x 64 unit lower triangles, and U12 of the
-// block's rows from them (trsm_block.hip).
+// Inverses of the 64 x 64 diagonal triangles of a packed LU of order n (unit
+// lower, or upper), and X <- T^-1 X for a block of nbo <= NB_OUT rows with
+// them (trsm_block.hip).
 template <typename T>
-int launch_block_linv(la_ctx *ctx, const T *Lblk, int64_t lda, int nbo, T *linv);
+int launch_block_inv(la_ctx *ctx, bool upper, const T *Tm, int64_t ldt, int64_t n, T *inv);
 template <typename T>
-int launch_u12_block(la_ctx *ctx, const T *Lblk, int64_t lda, const T *linv, int nbo, T *B,
-                     int64_t ldb, int64_t ncols);
+int launch_trsm_block(la_ctx *ctx, bool upper, const T *Tm, int64_t ldt, const T *inv, int nbo,
+                      T *B, int64_t ldb, int64_t ncols);
 
 }  // namespace lahip

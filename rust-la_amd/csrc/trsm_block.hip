@@ -1,5 +1,7 @@
-// U12 of the blocked LU: inverses of a block's 64 x 64 diagonal triangles
-// (k_block_linv) and X <- L11^-1 X over a whole outer block (k_u12_block).
+// Triangular solves with a block of up to 256 rows and many or few columns:
+// inverses of its 64 x 64 diagonal triangles (k_block_inv) and X <- T^-1 X
+// over the whole block (k_trsm_block).  Used for U12 of the blocked LU, and
+// with a GEMM per block for solves with several right-hand sides.
 #include "lu_device.hpp"
 
 namespace lahip {
@@ -20,34 +22,40 @@ template <> struct Mfma16<float> {
     }
 };
 
-// L11^-1 of the block's 64 x 64 diagonal triangles (one workgroup each), for
-// U12, from the factored block (Lblk, nbo columns): 64 x 64 at
-// linv + b * 64 * 64, zero outside the nb x nb triangle.
+// Inverses of the 64 x 64 diagonal triangles (one workgroup each) of a packed
+// LU whose first nbo columns start at Tm: of L (unit diagonal) or, UPPER, of
+// U, which is inverted as its transpose.  64 x 64 at inv + b * 64 * 64, zero
+// outside the nb x nb triangle.
 // By doubling: the four 16 x 16 diagonal inverses, one per wave by
 // substitution, then [X11 0; -X22 L21 X11, X22] for the two 32 x 32 blocks
 // and for the whole, on MFMA.  It sits on the LU's critical path between a
 // block and the next one's update.  One lane per column of the whole
 // triangle, 2016 unrolled FMAs, took 35 us, most of it waiting for
 // instructions (code that runs once per launch); this takes 6.
-template <typename T>
+template <typename T, bool UPPER>
 __global__ __launch_bounds__(256)
-void k_block_linv(const T *Lblk, int64_t lda, int nbo, T *linv)
+void k_block_inv(const T *Tm, int64_t ldt, int64_t nbo, T *inv)
 {
     typedef typename Mfma16<T>::acc_t acc_t;
     constexpr int LS = NB_IN + 4;
-    __shared__ T L[NB_IN][LS], X[NB_IN][LS], W[32][LS];
+    __shared__ T L[NB_IN][LS], X[NB_IN][LS], W[32][LS], rd[NB_IN];
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lhi = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nb = min(NB_IN, nbo - (int)blockIdx.x * NB_IN);
-    const T *src = Lblk + (int64_t)blockIdx.x * NB_IN * (lda + 1);
+    const int nb = (int)min((int64_t)NB_IN, nbo - (int64_t)blockIdx.x * NB_IN);
+    const T *src = Tm + (int64_t)blockIdx.x * NB_IN * (ldt + 1);
     T v[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-        v[k] = src[(int64_t)min(wave + 4 * k, nb - 1) * lda + min(lane, nb - 1)];
+        v[k] = src[(int64_t)min(wave + 4 * k, nb - 1) * ldt + min(lane, nb - 1)];
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         const int i = wave + 4 * k;
-        L[i][lane] = (i < nb && lane < i) ? v[k] : T(0);
+        if (UPPER) {
+            L[lane][i] = (lane < nb && i < lane) ? v[k] : T(0);
+            if (lane == i) rd[i] = i < nb ? T(1) / v[k] : T(1);
+        } else {
+            L[i][lane] = (i < nb && lane < i) ? v[k] : T(0);
+        }
         X[i][lane] = T(0);
     }
     __syncthreads();
@@ -59,7 +67,7 @@ void k_block_linv(const T *Lblk, int64_t lda, int nbo, T *linv)
             T s = l16 == i ? T(1) : T(0);
 #pragma unroll
             for (int t = 0; t < i; ++t) s -= L[d0 + i][d0 + t] * x[t];
-            x[i] = s;
+            x[i] = UPPER ? s * rd[d0 + i] : s;
         }
         if (lane < 16)
 #pragma unroll
@@ -95,29 +103,29 @@ void k_block_linv(const T *Lblk, int64_t lda, int nbo, T *linv)
 #pragma unroll
     for (int r = 0; r < 4; ++r) X[32 + ti + Mfma16<T>::drow(lhi, r)][tj + l16] = -x[r];
     __syncthreads();
-    T *out = linv + (size_t)blockIdx.x * NB_IN * NB_IN;
+    T *out = inv + (size_t)blockIdx.x * NB_IN * NB_IN;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         const int i = wave + 4 * k;
-        out[i * NB_IN + lane] = (i < nb && lane < nb) ? X[i][lane] : T(0);
+        out[i * NB_IN + lane] = (i < nb && lane < nb) ? (UPPER ? X[lane][i] : X[i][lane]) : T(0);
     }
 }
 
-// U12 for an outer block of nbo <= NB_OUT rows in one pass.  Each workgroup
-// keeps sixteen columns of A12 in LDS and runs the block forward substitution
-// on MFMA, sixteen rows of a 64-row panel per wave: for each panel b,
-// Y = X_b - sum_{k<b} L_bk X_k, then X_b = Linv_b Y (the panel's inverse,
-// from k_block_linv or the panel kernel), with L_bk read from the factored
-// block (Lblk = A + K0 * lda + K0).  The operands of L are loaded from memory
-// in fragment layout (a lane takes four consecutive k of every sixteen) one
-// 64 x 64 stage ahead, and none depends on X.
-// Bound by the chain of ten stages and their latency: it precedes the next
-// block's update on the LU's critical path.  256 columns take 16 us in FP64
-// (47 with the products on FMAs from LDS) and 13 in FP32 (36).
-template <typename T>
+// X <- T^-1 X (nbo <= NB_OUT rows, ncols columns at B) for the unit lower or,
+// UPPER, the upper triangle of the packed LU block at Tm, in one pass.  Each
+// workgroup keeps sixteen columns in LDS and substitutes block by block on
+// MFMA, sixteen rows of a 64-row panel per wave: for each panel b in order,
+// Y = X_b - sum of T_bk X_k over the panels k done, then X_b = inv(T_bb) Y
+// (inv: k_block_inv's or the LU panel kernel's).  The operands of T are
+// loaded from memory in fragment layout (a lane takes four consecutive k of
+// every sixteen) one 64 x 64 stage ahead, and none depends on X.
+// Bound by the chain of ten stages and their latency: as U12 it precedes the
+// next block's update on the LU's critical path.  256 columns take 16 us in
+// FP64 (47 with the products on FMAs from LDS) and 13 in FP32 (36).
+template <typename T, bool UPPER>
 __global__ __launch_bounds__(256)
-void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ linv, int nbo,
-                 T *B, int64_t ldb, int ncols)
+void k_trsm_block(const T *__restrict__ Tm, int64_t ldt, const T *__restrict__ inv, int nbo,
+                  T *B, int64_t ldb, int ncols)
 {
     typedef typename Mfma16<T>::acc_t acc_t;
     constexpr int CW = 16, XS = CW + 4;         // four lane groups in different banks
@@ -125,16 +133,29 @@ void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ 
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lhi = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c0 = blockIdx.x * CW, nb = (nbo + 63) / 64;
-    // stage (b, k): k < b is L_bk, k == b the inverse of panel b
+    // panels in order: at(s) is the s-th; stage (s, t): t < s is T_at(s),at(t),
+    // t == s the inverse of panel at(s)
+    auto at = [&](int s) __attribute__((always_inline)) { return UPPER ? nb - 1 - s : s; };
     T cur[16], nxt[16];
-    auto load = [&](T (&a)[16], int b, int k) __attribute__((always_inline)) {
-        const int row = min(16 * wave + l16, nbo - 64 * b - 1);
-        const T *src = (k < b ? Lblk + (int64_t)(64 * b + row) * lda + 64 * k
-                              : linv + (size_t)b * NB_IN * NB_IN + row * NB_IN) + 4 * lhi;
+    auto load = [&](T (&a)[16], int s, int t) __attribute__((always_inline)) {
+        const int b = at(s), k = at(t), row = min(16 * wave + l16, nbo - 64 * b - 1);
+        const T *src = (t < s ? Tm + (int64_t)(64 * b + row) * ldt + 64 * k
+                              : inv + (size_t)b * NB_IN * NB_IN + row * NB_IN) + 4 * lhi;
+        if (UPPER && t < s && 64 * k + 64 > nbo) {      // the ragged last panel's columns
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) a[4 * q + e] = src[16 * q + e];
+                for (int e = 0; e < 4; ++e) {
+                    const int c = 64 * k + 16 * q + 4 * lhi + e;
+                    a[4 * q + e] = src[min(16 * q + e, nbo - 1 - 64 * k - 4 * lhi)];
+                    if (c >= nbo) a[4 * q + e] = T(0);
+                }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[4 * q + e] = src[16 * q + e];
+        }
     };
     load(cur, 0, 0);
     {
@@ -144,7 +165,8 @@ void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ 
         for (int i = 0; i < 16; ++i)
             v[i] = B[(int64_t)min((tid >> 4) + 16 * i, nbo - 1) * ldb + col];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) X[(tid >> 4) + 16 * i][tid & 15] = v[i];
+        for (int i = 0; i < 16; ++i)
+            X[(tid >> 4) + 16 * i][tid & 15] = (tid >> 4) + 16 * i < nbo ? v[i] : T(0);
     }
     __syncthreads();
     auto mul = [&](const T (*x)[XS], acc_t acc) __attribute__((always_inline)) {
@@ -155,11 +177,12 @@ void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ 
                 acc = Mfma16<T>::op(cur[4 * q + e], x[16 * q + 4 * lhi + e][l16], acc);
         return acc;
     };
-    for (int b = 0; b < nb; ++b) {
+    for (int s = 0; s < nb; ++s) {
+        const int b = at(s);
         acc_t acc = {0, 0, 0, 0};
-        for (int k = 0; k < b; ++k) {
-            load(nxt, b, k + 1);
-            acc = mul(X + 64 * k, acc);
+        for (int t = 0; t < s; ++t) {
+            load(nxt, s, t + 1);
+            acc = mul(X + 64 * at(t), acc);
 #pragma unroll
             for (int i = 0; i < 16; ++i) cur[i] = nxt[i];
         }
@@ -169,14 +192,14 @@ void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ 
             Y[i][l16] = X[64 * b + i][l16] - acc[r];
         }
         __syncthreads();
-        if (b + 1 < nb) load(nxt, b + 1, 0);
+        if (s + 1 < nb) load(nxt, s + 1, 0);
         acc = mul(Y, acc_t{0, 0, 0, 0});
 #pragma unroll
         for (int i = 0; i < 16; ++i) cur[i] = nxt[i];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = 64 * b + 16 * wave + Mfma16<T>::drow(lhi, r);
-            X[i][l16] = acc[r];
+            X[i][l16] = i < nbo ? acc[r] : T(0);
             if (i < nbo && c0 + l16 < ncols) B[(int64_t)i * ldb + c0 + l16] = acc[r];
         }
         __syncthreads();
@@ -184,31 +207,41 @@ void k_u12_block(const T *__restrict__ Lblk, int64_t lda, const T *__restrict__ 
 }
 
 template <typename T>
-int launch_block_linv(la_ctx *ctx, const T *Lblk, int64_t lda, int nbo, T *linv)
+int launch_block_inv(la_ctx *ctx, bool upper, const T *Tm, int64_t ldt, int64_t n, T *inv)
 {
-    hipLaunchKernelGGL(k_block_linv<T>, dim3((unsigned)ceil_div(nbo, NB_IN)), dim3(256), 0,
-                       ctx->stream, Lblk, lda, nbo, linv);
+    const dim3 grid((unsigned)ceil_div(n, NB_IN));
+    if (upper)
+        hipLaunchKernelGGL((k_block_inv<T, true>), grid, dim3(256), 0, ctx->stream, Tm, ldt, n,
+                           inv);
+    else
+        hipLaunchKernelGGL((k_block_inv<T, false>), grid, dim3(256), 0, ctx->stream, Tm, ldt, n,
+                           inv);
     LA_HIP_CHECK(ctx, hipGetLastError());
     return LA_OK;
 }
 
 template <typename T>
-int launch_u12_block(la_ctx *ctx, const T *Lblk, int64_t lda, const T *linv, int nbo, T *B,
-                     int64_t ldb, int64_t ncols)
+int launch_trsm_block(la_ctx *ctx, bool upper, const T *Tm, int64_t ldt, const T *inv, int nbo,
+                      T *B, int64_t ldb, int64_t ncols)
 {
     ProfScope ps(ctx, LA_K_TRSM, (double)nbo * nbo * ncols,
                  (double)sizeof(T) * (2.0 * nbo * ncols + (double)nbo * nbo));
-    hipLaunchKernelGGL(k_u12_block<T>, dim3((unsigned)ceil_div(ncols, 16)), dim3(256), 0,
-                       ctx->stream, Lblk, lda, linv, nbo, B, ldb, (int)ncols);
+    const dim3 grid((unsigned)ceil_div(ncols, 16));
+    if (upper)
+        hipLaunchKernelGGL((k_trsm_block<T, true>), grid, dim3(256), 0, ctx->stream, Tm, ldt, inv,
+                           nbo, B, ldb, (int)ncols);
+    else
+        hipLaunchKernelGGL((k_trsm_block<T, false>), grid, dim3(256), 0, ctx->stream, Tm, ldt,
+                           inv, nbo, B, ldb, (int)ncols);
     LA_HIP_CHECK(ctx, hipGetLastError());
     return LA_OK;
 }
 
-template int launch_block_linv<double>(la_ctx *, const double *, int64_t, int, double *);
-template int launch_block_linv<float>(la_ctx *, const float *, int64_t, int, float *);
-template int launch_u12_block<double>(la_ctx *, const double *, int64_t, const double *, int,
-                                      double *, int64_t, int64_t);
-template int launch_u12_block<float>(la_ctx *, const float *, int64_t, const float *, int, float *,
-                                     int64_t, int64_t);
+template int launch_block_inv<double>(la_ctx *, bool, const double *, int64_t, int64_t, double *);
+template int launch_block_inv<float>(la_ctx *, bool, const float *, int64_t, int64_t, float *);
+template int launch_trsm_block<double>(la_ctx *, bool, const double *, int64_t, const double *,
+                                       int, double *, int64_t, int64_t);
+template int launch_trsm_block<float>(la_ctx *, bool, const float *, int64_t, const float *, int,
+                                      float *, int64_t, int64_t);
 
 }  // namespace lahip

@@ -13,7 +13,7 @@
 // in flight - then solves its own 64 x 64 diagonal triangle with one lane
 // per row and publishes its slice of x through a per-block flag.
 // Arithmetic is FP64; the factor may be FP64 or FP32 (the refinement path).
-#include "la_common.hpp"
+#include "lu_device.hpp"
 
 namespace lahip {
 
@@ -388,108 +388,44 @@ int trsv_blocked(la_ctx *ctx, char uplo, bool trans, bool unit, int64_t n, const
     return set_error(ctx, LA_ERR_ARG, "trsv: unsupported triangle");
 }
 
-// ------------------------------------------- many right-hand sides (TRSM)
-// For nrhs > NR the substitution becomes a blocked TRSM on the FP64 MFMA
-// GEMM: the 64 x 64 diagonal blocks are inverted once (one workgroup each,
-// in parallel), then, in dependency order, per super-block of eight blocks
-//   per block b:  Y = inv(T_bb) X_b;  X_(rest of super-block) -= T_.,b Y;  X_b = Y
-//   then          X_(rest of the triangle) -= T_.,super-block X_super-block
-// (right-looking: the update of the remaining rows is one GEMM of K = 512,
-// which runs the MFMA kernel far closer to its peak than eight of K = 64).
-template <int MODE, typename TF>
-__global__ __launch_bounds__(256)
-void k_diag_inverses(int n, const TF *__restrict__ Tm, int64_t ldt, double *Dinv)
-{
-    __shared__ double Ts[TB][TB + 1];
-    __shared__ double Xi[TB][TB + 1];
-    __shared__ double part[4][TB];
-    const int b = blockIdx.x, r0 = b * TB, rb = min(TB, n - r0), tid = threadIdx.x;
-    TF dv[TB * TB / 256];
-#pragma unroll
-    for (int k = 0; k < TB * TB / 256; ++k) {
-        const int e = tid + 256 * k, a = e / TB, c = e - a * TB;
-        dv[k] = Tm[(int64_t)(r0 + min(a, rb - 1)) * ldt + r0 + min(c, rb - 1)];
-    }
-#pragma unroll
-    for (int k = 0; k < TB * TB / 256; ++k) {
-        const int e = tid + 256 * k, a = e / TB, c = e - a * TB;
-        Ts[a][c] = (a < rb && c < rb) ? (double)dv[k] : 0.0;
-    }
-    __syncthreads();
-    invert_diag_block<MODE>(Ts, rb, Xi, part);
-    __syncthreads();
-    double *out = Dinv + (size_t)b * TB * TB;
-    for (int e = tid; e < TB * TB; e += blockDim.x) out[e] = Xi[e / TB][e % TB];
-}
-
-__global__ void k_copy_rows(int64_t rows, int64_t cols, const double *src, int64_t lds,
-                            double *dst, int64_t ldd)
-{
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= rows * cols) return;
-    const int64_t r = e / cols, c = e - r * cols;
-    dst[r * ldd + c] = src[r * lds + c];
-}
-
-// X (n x nrhs, ld ldx) <- T^-1 X for the LU triangles ('L' unit lower,
-// 'U' upper) of a packed FP64 factor.
+// ------------------------------------------ several right-hand sides (TRSM)
+// X (n x nrhs, ld ldx) <- T^-1 X for the LU triangles ('L' unit lower, 'U'
+// upper) of a packed FP64 factor.  The 64 x 64 diagonal blocks are inverted
+// once, in parallel; then, in dependency order, each 256-row block is solved
+// in one launch (trsm_block.hip) and one GEMM of K = 256 takes its rows out of
+// every row still to be solved.  k_trsv passes x from workgroup to workgroup
+// once per 64 rows and is bound by that exchange, which grows with the
+// right-hand sides: both triangles of n = 8192 with 16 take it 7.0 ms, of
+// n = 1500 with 7 0.84 ms, against 2.8 and 0.4 here.  With one right-hand side
+// k_trsv wins (TRSM_MIN_RHS); it also serves up to NR when the workspace limit
+// has no room for the inverses.
 int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ldt, int64_t nrhs,
                  double *X, int64_t ldx)
 {
     if (n <= 0 || nrhs <= 0) return LA_OK;
-    const int64_t nblocks = ceil_div(n, TB);
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t dbytes = al((size_t)nblocks * TB * TB * 8), ybytes = al((size_t)TB * nrhs * 8);
-    void *base = nullptr;
-    int st = ws_get(ctx, WS_LP, dbytes + ybytes, &base);
-    if (st) return st;
-    double *Dinv = (double *)base, *Y = (double *)((char *)base + dbytes);
+    if (n > INT32_MAX || nrhs > INT32_MAX) return set_error(ctx, LA_ERR_ARG, "trsm: too large");
     const bool lower = uplo == 'L';
-    if (lower)
-        hipLaunchKernelGGL((k_diag_inverses<MODE_LU_FWD, double>), dim3((unsigned)nblocks),
-                           dim3(256), 0, ctx->stream, (int)n, Tm, ldt, Dinv);
-    else
-        hipLaunchKernelGGL((k_diag_inverses<MODE_LU_BWD, double>), dim3((unsigned)nblocks),
-                           dim3(256), 0, ctx->stream, (int)n, Tm, ldt, Dinv);
-    LA_HIP_CHECK(ctx, hipGetLastError());
-    constexpr int64_t SBB = 8;                 // blocks per super-block
-    const int64_t nsuper = ceil_div(nblocks, SBB);
-    for (int64_t ss = 0; ss < nsuper; ++ss) {
-        const int64_t sb = lower ? ss : nsuper - 1 - ss;
-        const int64_t b_lo = sb * SBB, b_hi = std::min(nblocks, b_lo + SBB);
-        const int64_t R0 = b_lo * TB, R1 = std::min<int64_t>(n, b_hi * TB);
-        for (int64_t s = 0; s < b_hi - b_lo; ++s) {
-            const int64_t b = lower ? b_lo + s : b_hi - 1 - s;
-            const int64_t r0 = b * TB, rb = std::min<int64_t>(TB, n - r0);
-            double *Xb = X + r0 * ldx;
-            if ((st = gemm_rm<double>(ctx, rb, nrhs, rb, 1.0, Dinv + (size_t)b * TB * TB, TB, Xb,
-                                      ldx, 0.0, Y, nrhs, false, false)))
-                return st;
-            // the rows of this super-block still to be solved
-            if (lower && r0 + rb < R1) {
-                if ((st = gemm_rm<double>(ctx, R1 - r0 - rb, nrhs, rb, -1.0,
-                                          Tm + (r0 + rb) * ldt + r0, ldt, Y, nrhs, 1.0,
-                                          X + (r0 + rb) * ldx, ldx, false, false)))
-                    return st;
-            } else if (!lower && r0 > R0) {
-                if ((st = gemm_rm<double>(ctx, r0 - R0, nrhs, rb, -1.0, Tm + R0 * ldt + r0, ldt, Y,
-                                          nrhs, 1.0, X + R0 * ldx, ldx, false, false)))
-                    return st;
-            }
-            hipLaunchKernelGGL(k_copy_rows, dim3((unsigned)ceil_div(rb * nrhs, 256)), dim3(256), 0,
-                               ctx->stream, rb, nrhs, (const double *)Y, nrhs, Xb, ldx);
-            LA_HIP_CHECK(ctx, hipGetLastError());
-        }
-        // every row outside the super-block, with the super-block's rows of X
-        if (lower && R1 < n) {
-            if ((st = gemm_rm<double>(ctx, n - R1, nrhs, R1 - R0, -1.0, Tm + R1 * ldt + R0, ldt,
-                                      X + R0 * ldx, ldx, 1.0, X + R1 * ldx, ldx, false, false)))
-                return st;
-        } else if (!lower && R0 > 0) {
-            if ((st = gemm_rm<double>(ctx, R0, nrhs, R1 - R0, -1.0, Tm + R0, ldt, X + R0 * ldx, ldx,
-                                      1.0, X, ldx, false, false)))
-                return st;
-        }
+    const size_t bytes = (size_t)ceil_div(n, TB) * TB * TB * 8;
+    void *base = nullptr;
+    int st;
+    if (nrhs <= NR) {
+        if (!(base = ws_try(ctx, WS_LP, bytes)))
+            return trsv_blocked<double>(ctx, uplo, false, lower, n, Tm, ldt, nrhs, X, ldx);
+    } else if ((st = ws_get(ctx, WS_LP, bytes, &base))) {
+        return st;
+    }
+    double *inv = (double *)base;
+    if ((st = launch_block_inv<double>(ctx, !lower, Tm, ldt, n, inv))) return st;
+    const int64_t nblk = ceil_div(n, NB_OUT);
+    for (int64_t s = 0; s < nblk; ++s) {
+        const int64_t R0 = (lower ? s : nblk - 1 - s) * NB_OUT, R1 = std::min<int64_t>(n, R0 + NB_OUT);
+        if ((st = launch_trsm_block<double>(ctx, !lower, Tm + R0 * (ldt + 1), ldt, inv + R0 * TB,
+                                            (int)(R1 - R0), X + R0 * ldx, ldx, nrhs)))
+            return st;
+        const int64_t r0 = lower ? R1 : 0, rows = lower ? n - R1 : R0;
+        if ((st = gemm_rm<double>(ctx, rows, nrhs, R1 - R0, -1.0, Tm + r0 * ldt + R0, ldt,
+                                  X + R0 * ldx, ldx, 1.0, X + r0 * ldx, ldx, false, false)))
+            return st;
     }
     return LA_OK;
 }
