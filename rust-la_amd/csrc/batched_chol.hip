@@ -17,21 +17,28 @@
 //      (the diagonal block's rows) and goes straight on to step 2 while
 //      waves 1-3 update the other row tiles, so the serial diagonal block
 //      is hidden behind the rest of the panel update;
-//   2. wave 0 factors the NB x NB diagonal block: lane r holds row r, the
-//      column being eliminated is always register 0 (rows rotate left one
-//      step per column) and column values are broadcast with readlane, so
-//      the block needs no barrier; then it solves this block of y;
+//   2. wave 0 factors the NB x NB diagonal block: lane r holds row r, column
+//      values are broadcast with readlane, so the block needs no barrier;
+//      then it solves this block of y;
 //   3. every row below solves against the diagonal block in registers
 //      (row per thread), the panel and the zeros right of the diagonal block
 //      go to L, the rows below update their part of b from registers;
 //   backward substitution block by block, last block first: one wave solves
 //   the transposed diagonal block with readlane broadcasts, then the block's
 //   rows of L are pushed into the part of y above it in one coalesced sweep.
+//
+// What bounds it: 20000 problems, n uniform in [8, 256], take 4.8 ms (5.9 with
+// the diagonal block rotating its registers every column and masking every
+// update, a library square root and division per column, and problem sizes
+// and pointers in vector registers): the instructions and the latency of the
+// panel steps, of which the serial diagonal block on one wave is the longest;
+// moving A and L once takes 1.6 ms.
 // L is both output and left-looking operand; it is written and re-read by
 // the same workgroup with a workgroup barrier in between.
 #include "la_common.hpp"
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 namespace lahip {
 
@@ -58,6 +65,35 @@ __device__ inline double cb_bcast(double v, int lane) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// sqrt(d) and its reciprocal, d the same in every lane.  In the middle of the
+// range by Goldschmidt's iteration from v_rsq_f64 (h -> 1/(2 sqrt d), g ->
+// sqrt d, both refined by e = 1/2 - h g; g finally corrected by its residual):
+// eight dependent operations instead of the thirty of sqrt() and a division,
+// on the serial path through a problem's columns.
+__device__ inline void cb_sqrt_rcp(double d, double &root, double &rcp)
+{
+    if (d > 1e-280 && d < 1e280) {
+        const double y = __builtin_amdgcn_rsq(d);
+        double g = d * y, h = 0.5 * y;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const double e = fma(-h, g, 0.5);
+            g = fma(g, e, g);
+            h = fma(h, e, h);
+        }
+        root = fma(fma(-g, g, d), h, g);
+        rcp = 2.0 * h;
+    } else {
+        root = sqrt(d);
+        rcp = 1.0 / root;
+    }
+}
+template <typename F, int... I>
+__device__ __forceinline__ void cb_for_each(F &&f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
 // NB: panel width; RTW: row tiles whose MFMA K loops run together (more
 // loads in flight per round trip against more registers)
 template <int NB, int CB_RTW>
@@ -65,7 +101,8 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
                                const double *__restrict__ bp, double *xp, int32_t *status,
                                CbLds &S)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lhi = lane >> 4;
     if (tid == 0) S.bad = 0;
     for (int i = tid; i < n; i += CB_NT) S.y[i] = bp[i];
@@ -81,8 +118,8 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
         // together (4 + 4*RTW independent loads per lane per 16-wide chunk).
         const int rt_n = (m + 15) >> 4;
         int asym = 0;
-        const bool okB = l16 < jb;
-        const double *pb = Lp + (int64_t)(J0 + min(l16, jb - 1)) * n;
+        // 32-bit offsets from the problem's (uniform) pointers: n <= CB_MAXN
+        const uint32_t pb = (uint32_t)((J0 + min(l16, jb - 1)) * n);
         auto update_tiles = [&](auto rtw_c, int base, int step) {
             constexpr int RTW = decltype(rtw_c)::value;
             for (int pass = 0;; ++pass) {
@@ -91,21 +128,19 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
 #pragma unroll
                 for (int i = 0; i < RTW; ++i) acc[i] = (d4_t){0.0, 0.0, 0.0, 0.0};
                 if (J0 > 0) {
-                    const double *pa[RTW];
-                    bool okA[RTW];
+                    uint32_t pa[RTW];
 #pragma unroll
                     for (int i = 0; i < RTW; ++i) {
                         const int rowA = J0 + 16 * (base + step * (RTW * pass + i)) + l16;
-                        okA[i] = rowA < n;
-                        pa[i] = Lp + (int64_t)min(rowA, n - 1) * n;
+                        pa[i] = (uint32_t)(min(rowA, n - 1) * n);
                     }
                     // k = k0 + 4*(lane/16) + s for MFMA step s, the same for A
                     // and B; J0 is a multiple of 8, so a K chunk of 16 may end
                     // inside the current panel (or past J0): those columns are
-                    // masked out.  KU chunks are loaded together before their
-                    // MFMAs: every load is unconditional from a clamped column
-                    // (< J0) of a clamped row, and out-of-range values are
-                    // zeroed afterwards.
+                    // masked out (in B alone: the clamped A is part of the same
+                    // row).  KU chunks are loaded together before their MFMAs,
+                    // unconditionally, from a clamped column (< J0) of a clamped
+                    // row: rows past n and columns past jb are not stored.
                     constexpr int KU = 4 / RTW;
                     for (int k0 = 0; k0 < J0; k0 += 16 * KU) {
                         double a[KU][RTW][4], b[KU][4];
@@ -114,23 +149,18 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
                             // J0 is a multiple of 4: kc..kc+3 all below J0 or none
                             const int kc = min(k0 + 16 * u + 4 * lhi, J0 - 4);
 #pragma unroll
-                            for (int s = 0; s < 4; ++s) b[u][s] = pb[kc + s];
+                            for (int s = 0; s < 4; ++s) b[u][s] = (Lp + s)[pb + (uint32_t)kc];
 #pragma unroll
                             for (int i = 0; i < RTW; ++i)
 #pragma unroll
-                                for (int s = 0; s < 4; ++s) a[u][i][s] = pa[i][kc + s];
+                                for (int s = 0; s < 4; ++s) a[u][i][s] = (Lp + s)[pa[i] + (uint32_t)kc];
                         }
+                        if (k0 + 16 * KU > J0) {
 #pragma unroll
-                        for (int u = 0; u < KU; ++u) {
-                            const bool kin = k0 + 16 * u + 4 * lhi < J0;
-#pragma unroll
-                            for (int s = 0; s < 4; ++s)
-                                if (!(okB && kin)) b[u][s] = 0.0;
-#pragma unroll
-                            for (int i = 0; i < RTW; ++i)
+                            for (int u = 0; u < KU; ++u)
 #pragma unroll
                                 for (int s = 0; s < 4; ++s)
-                                    if (!(okA[i] && kin)) a[u][i][s] = 0.0;
+                                    if (k0 + 16 * u + 4 * lhi >= J0) b[u][s] = 0.0;
                         }
 #pragma unroll
                         for (int u = 0; u < KU; ++u)
@@ -154,8 +184,8 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const int grc = J0 + min(16 * rt + lhi + 4 * r, m - 1);
-                            v[r] = Ap[(int64_t)grc * n + gcc];
-                            w[r] = Ap[(int64_t)gcc * n + grc];
+                            v[r] = Ap[(uint32_t)(grc * n + gcc)];
+                            w[r] = Ap[(uint32_t)(gcc * n + grc)];
                         }
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
@@ -176,34 +206,47 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
             // keep the compiler from moving the reads above the writes (LDS
             // executes one wave's operations in order)
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            // ---- 2. diagonal block, rows in registers (rotated)
+            // ---- 2. diagonal block, rows in registers
             double a[NB];
 #pragma unroll
             for (int c = 0; c < NB; ++c) a[c] = (lane < jb && c < jb) ? S.P[lane][c] : 0.0;
-#pragma unroll 1
-            for (int t = 0; t < NB; ++t) {
-                if (t < jb) {
-                    const double dd = cb_bcast(a[0], t);      // A[t][t] after the updates
-                    if (lane == 0 && dd <= 0.0) atomicOr(&S.bad, 2);
-                    const double d = sqrt(dd);
-                    const double rd = 1.0 / d;
-                    if (lane == 0) S.dinv[t] = rd;
-                    const double l = a[0] * rd;
-                    if (lane == t) a[0] = d;
-                    else if (lane > t) a[0] = l;
-                    // columns t+1..: lane r >= t+j subtracts L[r][t] L[t+j][t];
-                    // readlane indices stay below 32, masked lanes add zero
+            // Column t is register t % 8 of the first block of eight; after
+            // eight columns the blocks rotate, so the code is eight columns
+            // long and only blocks with columns still to come are updated.
+            // Entries right of the diagonal, and columns past jb, are scratch.
+            auto column = [&](auto c_c, int it) __attribute__((always_inline)) {
+                constexpr int c = decltype(c_c)::value;
+                const int t = 8 * it + c;
+                if (t >= jb) return;
+                const double dd = cb_bcast(a[c], t);          // A[t][t] after the updates
+                if (lane == 0 && dd <= 0.0) atomicOr(&S.bad, 2);
+                double d, rd;
+                cb_sqrt_rcp(dd, d, rd);
+                if (lane == 0) S.dinv[t] = rd;
+                const double l = a[c] * rd;
+                a[c] = lane == t ? d : l;
+                // readlane indices stay below 16
 #pragma unroll
-                    for (int j = 1; j < NB; ++j) {
-                        const double ltj = cb_bcast(l, t + j);
-                        const double lm = (lane >= t + j && t + j < jb) ? l : 0.0;
-                        a[j] = fma(-lm, ltj, a[j]);
+                for (int b = 0; b < NB / 8; ++b)
+                    if (b < NB / 8 - it) {
+#pragma unroll
+                        for (int j = 8 * b; j < 8 * b + 8; ++j)
+                            if (j > c) a[j] = fma(-l, cb_bcast(l, 8 * it + j), a[j]);
                     }
-                }
-                const double a0 = a[0];
+            };
+#pragma unroll 1
+            for (int it = 0; it < NB / 8; ++it) {
+                cb_for_each([&](auto c_c) __attribute__((always_inline)) { column(c_c, it); },
+                            std::make_integer_sequence<int, 8>{});
+                if (NB > 8) {
+                    double h[8];
 #pragma unroll
-                for (int c = 0; c < NB - 1; ++c) a[c] = a[c + 1];
-                a[NB - 1] = a0;
+                    for (int c = 0; c < 8; ++c) h[c] = a[c];
+#pragma unroll
+                    for (int c = 0; c < NB - 8; ++c) a[c] = a[c + 8];
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) a[NB - 8 + c] = h[c];
+                }
             }
             if (lane < jb) {
 #pragma unroll
@@ -242,16 +285,17 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
                     x[c] = s * S.dinv[c];
                 }
             }
-            double *lr = Lp + (int64_t)(J0 + r) * n + J0;
+            double *const lj = Lp + J0;
+            const uint32_t lr = (uint32_t)((J0 + r) * n);
 #pragma unroll
             for (int c = 0; c < NB; ++c)
-                if (c < jb) lr[c] = x[c];
+                if (c < jb) (lj + c)[lr] = x[c];
         }
         // diagonal block rows, with the zeros of the upper triangle
-        for (int e = tid; e < jb * m; e += CB_NT) {
-            const int rr = e / m, c = e - rr * m;
-            Lp[(int64_t)(J0 + rr) * n + J0 + c] = (c < jb && c <= rr) ? S.P[rr][c] : 0.0;
-        }
+        for (int rr = wave; rr < jb; rr += 4)
+            for (int c = lane; c < m; c += 64)
+                Lp[(uint32_t)((J0 + rr) * n + J0 + c)] =
+                    (c < jb && c <= rr) ? S.P[rr][min(c, NB - 1)] : 0.0;
         __syncthreads();
         if (r < m) {
             double s = 0.0;
@@ -277,12 +321,12 @@ __device__ __forceinline__ void chol_solve_one(int n, const double *__restrict__
         const bool push = c < J0;
 #pragma unroll
         for (int rr = 0; rr < NB; ++rr)
-            lp[rr] = Lp[(int64_t)(J0 + min(rr, jb - 1)) * n + min(c, J0 > 0 ? J0 - 1 : 0)];
+            lp[rr] = Lp[(uint32_t)((J0 + min(rr, jb - 1)) * n + min(c, J0 > 0 ? J0 - 1 : 0))];
         if (wave == 0) {
             double colv[NB];          // lane c: column c of the diagonal block
 #pragma unroll
             for (int rr = 0; rr < NB; ++rr)
-                colv[rr] = Lp[(int64_t)(J0 + min(rr, jb - 1)) * n + J0 + min(lane, jb - 1)];
+                colv[rr] = Lp[(uint32_t)((J0 + min(rr, jb - 1)) * n + J0 + min(lane, jb - 1))];
             const double dgi = 1.0 / Lp[(int64_t)(J0 + min(lane, jb - 1)) * n + J0 + min(lane, jb - 1)];
             double xv = lane < jb ? S.y[J0 + lane] : 0.0;
 #pragma unroll
@@ -323,7 +367,8 @@ void k_chol_batched(int count, const int32_t *__restrict__ order, const int32_t 
     for (;;) {
         if (threadIdx.x == 0) S.prob = (int)atomicAdd(&queue[0], 1u);
         __syncthreads();
-        const int pi = S.prob;
+        // uniform: sizes and pointers of the problem stay in scalar registers
+        const int pi = __builtin_amdgcn_readfirstlane(S.prob);
         __syncthreads();
         if (pi >= count) break;
         const int prob = order[pi];
