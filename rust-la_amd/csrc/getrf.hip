@@ -1143,17 +1143,10 @@ struct LookAhead {
     bool tried = false;
 };
 
-// Two pairs: 8 CUs per XCD for the panel stream where every block goes to the
-// column-distributed kernel (narrow; at most 64 workgroups of one per CU), 12
-// where row-distributed panels run, which take as many CUs as they get.
-// Measured for 8 / 12: FP32-IR n = 16384 71.1 / 73.6 ms, FP64 LU n = 8192 +
-// 16 rhs 27.7 / 28.0 ms; FP64 LU n = 16384 (row-distributed above 8192 rows)
-// 114.4 / 98.9 ms.
-static const LookAhead *lookahead_streams(la_ctx *ctx, bool narrow)
+static const LookAhead *lookahead_streams(la_ctx *ctx)
 {
     static std::mutex mu;
-    static LookAhead la_all[2][16];
-    LookAhead *la = la_all[narrow];
+    static LookAhead la[16];
     const char *off = getenv("LAHIP_LOOKAHEAD");
     if (off && atoi(off) == 0) return nullptr;
     if (ctx->device < 0 || ctx->device >= 16 || ctx->num_cus < 16 || ctx->num_cus % 8 != 0)
@@ -1162,7 +1155,7 @@ static const LookAhead *lookahead_streams(la_ctx *ctx, bool narrow)
     LookAhead &l = la[ctx->device];
     if (!l.tried) {
         l.tried = true;
-        int per_xcd = narrow ? 8 : 12;
+        int per_xcd = 12;
         if (const char *e = getenv("LAHIP_PANEL_CUS_PER_XCD")) per_xcd = atoi(e);
         per_xcd -= per_xcd % 4;
         const int xcd_cus = ctx->num_cus / 8;
@@ -1225,6 +1218,7 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
         return set_error(ctx, LA_ERR_ARG, "getrf: extent too large");
     const int64_t kmax = m < n ? m : n;
     // outer block from which the look-ahead schedule runs (kmax: never)
+    const LookAhead *la = ext_ws ? nullptr : lookahead_streams(ctx);
     int64_t K0la = kmax;
     // Which blocks go to the column-distributed kernel: by their rows alone,
     // so that every schedule and entry point factors a block the same way.
@@ -1238,9 +1232,6 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     auto block_for = [&](int64_t K0) -> const BlockCfg * {
         return pub ? block_cfg<T>(m - K0, num_cus) : nullptr;
     };
-    const LookAhead *la =
-        ext_ws ? nullptr
-               : lookahead_streams(ctx, !lp && !exact && block_cfg<T>(m, num_cus) != nullptr);
     // panel workspace
     size_t slot_bytes = (size_t)2 * PANEL_MAXP * CAND_WORDS * sizeof(uint64_t);
     size_t row_bytes = 256;
