@@ -61,6 +61,12 @@ int ws_get(la_ctx *ctx, int id, size_t bytes, void **out) {
 
 void *ws_try(la_ctx *ctx, int id, size_t bytes) {
     void *p = nullptr;
+    if (ctx->ws[id].size < bytes) {
+        // growing allocates and synchronises, which would end a capture
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
+        if (cap != hipStreamCaptureStatusNone) return nullptr;
+    }
     const std::string before = ctx->last_error;
     if (ws_get(ctx, id, bytes, &p) == LA_OK) return p;
     (void)hipGetLastError();

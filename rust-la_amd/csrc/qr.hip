@@ -680,7 +680,7 @@ int qr_ws(la_ctx *ctx, int64_t m, int64_t n, int64_t wcols, QrWs &w)
     const size_t least = std::max((size_t)VT_MAXCHUNK * bw, (size_t)QRP_MAXP * QR_G_BYTES) + bw +
                          2 * QR_G_BYTES;
     w.pool_bytes = std::max(full, least);
-    void *base = ws_try(ctx, WS_QR, fixed + w.pool_bytes);
+    void *base = ctx->ws_limit > 0 ? nullptr : ws_try(ctx, WS_QR, fixed + w.pool_bytes);
     if (!base) {
         w.pool_bytes = least;
         int st = ws_get(ctx, WS_QR, fixed + least, &base);

@@ -397,8 +397,9 @@ int trsv_blocked(la_ctx *ctx, char uplo, bool trans, bool unit, int64_t n, const
 // once per 64 rows and is bound by that exchange, which grows with the
 // right-hand sides: both triangles of n = 8192 with 16 take it 7.0 ms, of
 // n = 1500 with 7 0.84 ms, against 2.8 and 0.4 here.  With one right-hand side
-// k_trsv wins (TRSM_MIN_RHS); it also serves up to NR when the workspace limit
-// has no room for the inverses.
+// k_trsv wins (TRSM_MIN_RHS); it also serves up to NR when a workspace limit is
+// set, under which the inverses could take the room of a later call, and when
+// they would have to be allocated inside a capture.
 int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ldt, int64_t nrhs,
                  double *X, int64_t ldx)
 {
@@ -409,7 +410,8 @@ int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ld
     void *base = nullptr;
     int st;
     if (nrhs <= NR) {
-        if (!(base = ws_try(ctx, WS_LP, bytes)))
+        const bool grow = ctx->ws[WS_LP].size < bytes;
+        if ((grow && ctx->ws_limit > 0) || !(base = ws_try(ctx, WS_LP, bytes)))
             return trsv_blocked<double>(ctx, uplo, false, lower, n, Tm, ldt, nrhs, X, ldx);
     } else if ((st = ws_get(ctx, WS_LP, bytes, &base))) {
         return st;
