@@ -1136,7 +1136,12 @@ static int launch_block_moves(la_ctx *ctx, T *A, int64_t lda, int64_t n, int64_t
 // a mask that leaves an XCD with no CU.
 // Cooperative launches ignore CU masks, which is why the masked panel is an
 // ordinary launch sized by masked_panel_rpl.  The streams live until the
-// process ends (the runtime allows only a few masked hardware queues).
+// process ends (the runtime allows only a few masked hardware queues).  One
+// pair serves every factorisation: 12 CUs per XCD (the default) is what the
+// row-distributed panels need (FP64 n = 16384: 99 ms, 114 with 8), and a second
+// pair of 8 for the factorisations whose blocks need only 64 CUs (FP32-IR
+// n = 16384: 71.1 against 73.6 ms) slows whichever pair a process uses second
+// by a tenth (BF16 + GMRES n = 16384 115 -> 126 ms, FP32-IR 62 -> 69 ms).
 struct LookAhead {
     hipStream_t panel = nullptr, update = nullptr;
     int panel_cus = 0;
