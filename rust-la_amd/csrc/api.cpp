@@ -394,7 +394,7 @@ static int getrs_device(la_ctx *ctx, int64_t m, int64_t n, const double *dLU, in
                         double *dX, int64_t ldx) {
     int st;
     if ((st = gather_rows(ctx, m, nx, dpiv, dB, ldb, dX, ldx))) return st;
-    if (nx >= TRSM_MIN_RHS && n >= TRSM_MIN_N) {     // many columns: MFMA TRSM
+    if (trsm_wins(n, nx)) {
         if ((st = trsm_blocked(ctx, 'L', n, dLU, ldlu, nx, dX, ldx))) return st;
         return trsm_blocked(ctx, 'U', n, dLU, ldlu, nx, dX, ldx);
     }

@@ -872,7 +872,7 @@ int qr_solve_device(la_ctx *ctx, int64_t m, int64_t n, const double *QR, int64_t
     hipLaunchKernelGGL(k_qr_copy, dim3((unsigned)ceil_div(n * nx, 256)), dim3(256), 0,
                        ctx->stream, (int)n, (int)nx, (const double *)Y, ldy, X, ldx);
     LA_HIP_CHECK(ctx, hipGetLastError());
-    if (nx >= TRSM_MIN_RHS && n >= TRSM_MIN_N) return trsm_blocked(ctx, 'U', n, R, n, nx, X, ldx);
+    if (trsm_wins(n, nx)) return trsm_blocked(ctx, 'U', n, R, n, nx, X, ldx);
     return trsv_blocked<double>(ctx, 'U', false, false, n, R, n, nx, X, ldx);
 }
 
