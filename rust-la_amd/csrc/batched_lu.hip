@@ -104,6 +104,11 @@ template <typename T> __device__ inline void bl_wave_best(uint64_t &key, uint32_
     key = ((uint64_t)hi << 32) | lo;
     q = mq;
 }
+__device__ inline int bl_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline int64_t bl_uniform(int64_t v) {
+    const uint32_t lo = (uint32_t)bl_uniform((int)v), hi = (uint32_t)bl_uniform((int)(v >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
 template <typename F, int... I>
 __device__ __forceinline__ void bl_for_each(F &&f, std::integer_sequence<int, I...>) {
     (f(std::integral_constant<int, I>{}), ...);
@@ -127,6 +132,8 @@ __device__ inline double bl_wave_sum(double v) {
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
     return v;
 }
+
+__device__ inline double bl_abs_or_inf(double v) { return v == v ? fabs(v) : INFINITY; }
 
 // FP32 / FP64 MFMA, the accumulator row of its element r, and the K batch of
 // bl_rows_times
@@ -612,8 +619,11 @@ bl_rows_times(const T *__restrict__ mrow, const T *X, int ldx, int g, int j0, in
 // rows per wave; the diagonal tile is loaded (coalesced) before it, staged in
 // LDS and solved one row per lane with readlane broadcasts, each wave taking
 // right-hand sides c and c + 4 together so that their chains overlap.  The
-// upper tile's rows are scaled by the reciprocal of their diagonal once, so
-// the chain has no division (unless a reciprocal is not finite).
+// chain through the upper tile divides by its diagonal with div_rcp, three
+// dependent operations; a result that is not finite is formed again with
+// divisions.  (Rows scaled by their reciprocal ahead of the chain would
+// leave only the product in it, but u / d leaves the range of T where u x
+// and the quotient are ordinary numbers: columns of scales 1e-20 and 1e20.)
 template <typename T>
 __device__ void bl_trsv_lu(int n, const T *__restrict__ W, T *Y, int g, unsigned char *stg)
 {
@@ -662,19 +672,18 @@ __device__ void bl_trsv_lu(int n, const T *__restrict__ W, T *Y, int g, unsigned
                         if (i > k) { y0 -= l * a; y1 -= l * b; }
                     }
             } else {
-                const T d = D[i][i], rd = (T)1 / d;
-                if (!__any(!(fabs(rd) < (T)INFINITY))) {
-                    y0 *= rd;
-                    y1 *= rd;
+                const T d = D[i][i], rd = (T)1 / d, s0 = y0, s1 = y1;
 #pragma unroll
-                    for (int k = 0; k < 64; ++k) row[k] *= rd;
-#pragma unroll
-                    for (int k = 63; k >= 1; --k)
-                        if (k < bs) {
-                            const T a = bl_bcast(y0, k), b = bl_bcast(y1, k);
-                            if (i < k) { y0 -= row[k] * a; y1 -= row[k] * b; }
-                        }
-                } else {
+                for (int k = 63; k >= 0; --k)
+                    if (k < bs) {
+                        const T q0 = div_rcp(y0, d, rd), q1 = div_rcp(y1, d, rd);
+                        if (i == k) { y0 = q0; y1 = q1; }
+                        const T a = bl_bcast(y0, k), b = bl_bcast(y1, k);
+                        if (i < k) { y0 -= row[k] * a; y1 -= row[k] * b; }
+                    }
+                if (__any(!(fabs(y0) < (T)INFINITY && fabs(y1) < (T)INFINITY))) {
+                    y0 = s0;
+                    y1 = s1;
 #pragma unroll 1
                     for (int k = bs - 1; k >= 0; --k) {
                         if (i == k) { y0 = y0 / d; y1 = y1 / d; }
@@ -694,8 +703,9 @@ __device__ void bl_trsv_lu(int n, const T *__restrict__ W, T *Y, int g, unsigned
 
 // ----------------------------------------------------------- refinement
 // r = b - A x (FP64) for the rows in pivot order; Y[i][c] = r[perm[i]][c]
-// in working precision; L.rn[c] = max |r_c|.  Sixteen rows per wave at a time
-// on FP64 MFMA.
+// in working precision; L.rn[c] = max |r_c|, a NaN counted as infinite (fmax
+// would drop it, and a NaN residual would pass for none).  Sixteen rows per
+// wave at a time on FP64 MFMA.
 template <int MODE>
 __device__ void bl_residual(int n, int nrhs, int c0, int g, bool first,
                             const double *__restrict__ Ap, const double *__restrict__ Bp,
@@ -732,7 +742,7 @@ __device__ void bl_residual(int n, int nrhs, int c0, int g, bool first,
             if (i < n && l16 < g) {
                 const double v = bv[r] - acc[r];
                 Y[i * g + l16] = (T)v;
-                rmax = fmax(rmax, fabs(v));
+                rmax = fmax(rmax, bl_abs_or_inf(v));
             }
         }
     }
@@ -746,7 +756,7 @@ __device__ void bl_residual(int n, int nrhs, int c0, int g, bool first,
     __syncthreads();
 }
 
-// x += Y (columns c0..c0+g-1); L.xn[c] = max |x_c| afterwards
+// x += Y (columns c0..c0+g-1); L.xn[c] = max |x_c| afterwards (NaN: infinite)
 template <int MODE>
 __device__ void bl_update_x(int n, int nrhs, int c0, int g, double *Xp, BlLds<MODE> &L,
                             bool first)
@@ -764,7 +774,7 @@ __device__ void bl_update_x(int n, int nrhs, int c0, int g, double *Xp, BlLds<MO
         *xp = v;
 #pragma unroll
         for (int q = 0; q < BL_MAXRHS; ++q)
-            if (q == c) xm[q] = fmax(xm[q], fabs(v));
+            if (q == c) xm[q] = fmax(xm[q], bl_abs_or_inf(v));
     }
 #pragma unroll
     for (int c = 0; c < BL_MAXRHS; ++c) {
@@ -845,12 +855,15 @@ void k_lu_ir_batched(int count, const int32_t *__restrict__ order, const int32_t
     for (;;) {
         if (threadIdx.x == 0) L.prob = (int)atomicAdd(&queue[0], 1u);
         __syncthreads();
-        // uniform: sizes and pointers of the problem stay in scalar registers
+        // uniform: the problem's sizes and pointers stay in scalar registers and
+        // its loops are scalar branches.  As vector values they were the first
+        // to be spilled, and a spill at the end of a divergent branch was
+        // placed ahead of the restore of exec, which keeps lane 0's value only.
         const int pi = __builtin_amdgcn_readfirstlane(L.prob);
         __syncthreads();
         if (pi >= count) break;
-        const int prob = order[pi];
-        const int n = nvec[prob], nrhs = rhsvec[prob];
+        const int prob = bl_uniform(order[pi]);
+        const int n = bl_uniform(nvec[prob]), nrhs = bl_uniform(rhsvec[prob]);
         if (n <= 0 || n > BL_MAXN || nrhs <= 0 || nrhs > BL_MAXRHS) {
             if (threadIdx.x == 0) {
                 status[prob] = LA_ERR_SHAPE;
@@ -859,11 +872,11 @@ void k_lu_ir_batched(int count, const int32_t *__restrict__ order, const int32_t
             }
             continue;
         }
-        const double *Ap = A + offA[prob];
-        const double *Bp = B + offB[prob];
-        double *Xp = X + offB[prob];
-        typename BlCfg<MODE>::T *Wp = Wbuf + offW[prob];
-        int *perm = permbuf + offN[prob];
+        const double *Ap = A + bl_uniform(offA[prob]);
+        const double *Bp = B + bl_uniform(offB[prob]);
+        double *Xp = X + bl_uniform(offB[prob]);
+        typename BlCfg<MODE>::T *Wp = Wbuf + bl_uniform(offW[prob]);
+        int *perm = permbuf + bl_uniform(offN[prob]);
         double anorm, amax;
         bl_convert<MODE>(n, Ap, Wp, perm, L, anorm, amax);
         float uscale = 1.0f;

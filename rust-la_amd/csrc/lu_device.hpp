@@ -67,6 +67,18 @@ __device__ inline int ld_status(const int32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// y / d from rd = 1 / d: the product, corrected by its residual to what a
+// division gives (a last bit apart where the residual is subnormal).  Not
+// finite where y, d, rd or the quotient is not: there the caller divides.
+__device__ inline double div_rcp(double y, double d, double rd) {
+    const double q = y * rd;
+    return fma(fma(-q, d, y), rd, q);
+}
+__device__ inline float div_rcp(float y, float d, float rd) {
+    const float q = y * rd;
+    return fmaf(fmaf(-q, d, y), rd, q);
+}
+
 constexpr int BLK_MAP_MAX = 2 * NB_OUT;         // rows a block's swaps can move
 
 // A layout of the column-distributed block kernel (getrf_block.hip).

@@ -51,3 +51,58 @@ def test_scaled_permutations_are_exact(tctx, torch_cuda, prec):
     bt["B"].copy_(torch.from_numpy(b))
     (x, st, it, be), = solve_batch(torch, tctx, bt, prec)
     assert (st == 0).all() and np.array_equal(x, want) and (be == 0).all()
+
+
+def _solve_list(torch, ctx, prec, problems):
+    sizes, nrhs = [a.shape[0] for a, _ in problems], [b.shape[1] for _, b in problems]
+    bt = make_batch(torch, ctx, sizes, nrhs)
+    bt["A"].copy_(torch.from_numpy(np.concatenate([a.ravel() for a, _ in problems])))
+    bt["B"].copy_(torch.from_numpy(np.concatenate([b.ravel() for _, b in problems])))
+    (x, st, it, be), = solve_batch(torch, ctx, bt, prec)
+    return [x[o:o + n * r].reshape(n, r) for o, n, r in zip(bt["offB"], sizes, nrhs)], st, be
+
+
+# Columns of very different scales: u / d of the back substitution is outside
+# the range of the working precision where u x and the quotients are ordinary.
+@pytest.mark.parametrize("prec,small,large", [(la_hip.PREC_FP64, 1e-160, 1e160),
+                                              (la_hip.PREC_FP32, 1e-25, 1e15),
+                                              (la_hip.PREC_FP16, 1e-25, 1e15)])
+def test_back_substitution_range(tctx, torch_cuda, prec, small, large):
+    a = np.array([[small, large], [0.0, 1.0]])
+    t = 1e-5 * small                        # x = [1 - 1e-5 large, t]
+    (x, y), st, be = _solve_list(torch_cuda, tctx, prec, [(a, np.array([[small], [0.0]])),
+                                                          (a, np.array([[small], [t]]))])
+    assert (st == 0).all() and np.array_equal(x, [[1.0], [0.0]])
+    # two roundings of each operand and one per operation in working precision
+    u = 2.0 ** -53 if prec == la_hip.PREC_FP64 else 2.0 ** -24
+    want = np.array([[1.0 - 1e-5 * large], [t]])
+    assert np.abs(y / want - 1.0).max() <= 8 * u
+
+
+@pytest.mark.parametrize("prec,n,s", [(la_hip.PREC_FP64, 70, 160), (la_hip.PREC_FP32, 70, 20),
+                                      (la_hip.PREC_FP16, 24, 20)])
+def test_column_scales(tctx, torch_cuda, prec, n, s):
+    rng = np.random.default_rng(n)
+    r = rng.uniform(-1.0, 1.0, (n, n)) + 4 * np.sqrt(n) * np.eye(n)
+    scale = np.where(rng.random(n) < 0.5, 10.0 ** -s, 10.0 ** s)
+    b = rng.uniform(-1.0, 1.0, (n, 3))
+    (x,), st, be = _solve_list(torch_cuda, tctx, prec, [(r * scale, b)])
+    assert (st == 0).all()
+    want = np.linalg.solve(r, b)
+    # kappa_inf(r) < 6 and growth 1: at most 3 n u kappa for one solve
+    u = 2.0 ** -53 if prec == la_hip.PREC_FP64 else 2.0 ** -24
+    assert np.abs(x * scale[:, None] - want).max() <= 18 * n * u * np.abs(want).max()
+
+
+# A NaN is no small residual: eta is not 0, and refinement does not converge.
+@pytest.mark.parametrize("prec", PRECS)
+def test_nan_right_hand_side(tctx, torch_cuda, prec):
+    rng = np.random.default_rng(1)
+    a = rng.uniform(-1.0, 1.0, (40, 40)) + 8 * np.eye(40)
+    b = rng.uniform(-1.0, 1.0, (40, 2))
+    bad = b.copy()
+    bad[7, 1] = np.nan
+    (x, y), st, be = _solve_list(torch_cuda, tctx, prec, [(a, bad), (a, b)])
+    assert be[0] > 1.0 and be[1] <= 1e-14
+    assert st[0] == (0 if prec == la_hip.PREC_FP64 else la_hip.LA_NOT_CONVERGED) and st[1] == 0
+    assert eta_of(a, y, b) <= 1e-14
