@@ -122,10 +122,13 @@ __device__ inline double bl_bcast(double v, int lane) {
     const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
+// largest of the wave's values, which are not negative and not NaN: their
+// bits order as they do
 __device__ inline double bl_wave_max(double v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v = fmax(v, __shfl_xor(v, m));
-    return v;
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t hi = (uint32_t)(b >> 32), mhi = wave_max_u32(hi);
+    const uint32_t mlo = wave_max_u32(hi == mhi ? (uint32_t)b : 0u);
+    return __longlong_as_double((long long)(((uint64_t)mhi << 32) | mlo));
 }
 __device__ inline double bl_wave_sum(double v) {
 #pragma unroll
@@ -195,7 +198,10 @@ __device__ void bl_convert(int n, const double *__restrict__ Ap,
     }
     for (int i = tid; i < n; i += BL_NT) perm[i] = i;
     vmax = bl_wave_max(vmax);
-    if (lane == 0) { L.red[wave] = rs_max; L.red[4 + wave] = vmax; }
+    // the same values from every lane: a branch here is where the compiler
+    // placed spills ahead of the restore of exec
+    L.red[wave] = rs_max;
+    L.red[4 + wave] = vmax;
     __syncthreads();
     anorm = fmax(fmax(L.red[0], L.red[1]), fmax(L.red[2], L.red[3]));
     amax = fmax(fmax(L.red[4], L.red[5]), fmax(L.red[6], L.red[7]));
@@ -508,12 +514,14 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
 #pragma unroll
                         for (int r = 0; r < 4; ++r) cv[g][r] = W[off[r] + (uint32_t)col];
                     }
-                    acc_t acc[G];
-#pragma unroll
-                    for (int g = 0; g < G; ++g) acc[g] = acc_t{0, 0, 0, 0};
+                    // the products of sixteen (32) k are summed, then taken
+                    // from C: the sum of all 64 outgrows C and rounds coarser
 #pragma unroll
                     for (int q = 0; q < BL_KO; q += KS)
                         if (q < kd) {
+                            acc_t acc[G];
+#pragma unroll
+                            for (int g = 0; g < G; ++g) acc[g] = acc_t{0, 0, 0, 0};
                             if constexpr (MODE == LA_PREC_FP16) {
 #pragma unroll
                                 for (int g = 0; g < G; ++g)
@@ -532,16 +540,19 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
                                             ustg[(q + 4 * lhi + e) * US + 16 * (ct0 + g) + l16],
                                             acc[g]);
                             }
+#pragma unroll
+                            for (int g = 0; g < G; ++g)
+#pragma unroll
+                                for (int r = 0; r < 4; ++r)
+                                    cv[g][r] -= MODE == LA_PREC_FP16 ? (T)(acc[g][r] * uinv) : acc[g][r];
                         }
 #pragma unroll
                     for (int g = 0; g < G; ++g) {
                         const int cl = 16 * (ct0 + g) + l16;
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const T d = MODE == LA_PREC_FP16 ? (T)(acc[g][r] * uinv) : acc[g][r];
+                        for (int r = 0; r < 4; ++r)
                             if (row0 + BlVec<T>::drow(lhi, r) < n && cl < cw)
-                                W[off[r] + (uint32_t)(cc0 + cl)] = cv[g][r] - d;
-                        }
+                                W[off[r] + (uint32_t)(cc0 + cl)] = cv[g][r];
                     }
                 }
             }
@@ -559,7 +570,9 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
 // are loaded while the KB before them are multiplied: these products are
 // bound by the way to memory (M is read once), and four rows at a time with
 // eight 4- or 8-byte loads in flight reached 1.2 (FP64) and 0.5 TB/s (FP32).
-// Four accumulators, one per sixteen columns of a batch, are added at the end.
+// The sum is short in depth, since it is the residual of the refinement: the
+// products of four columns, added pairwise to those of sixteen, which go to
+// four accumulators in turn.
 template <typename T>
 __device__ __forceinline__ typename BlVec<T>::acc_t
 bl_rows_times(const T *__restrict__ mrow, const T *X, int ldx, int g, int j0, int j1)
@@ -598,11 +611,13 @@ bl_rows_times(const T *__restrict__ mrow, const T *X, int ldx, int g, int j0, in
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             if (j + 16 * c < j1) {
+                acc_t t[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const T x = xc[min(j + 16 * c + 4 * lhi + e, j1 - 1) * ldx];
-                    acc[c & 3] = BlVec<T>::mfma(v[c][e], x, acc[c & 3]);
+                    t[e] = BlVec<T>::mfma(v[c][e], x, acc_t{0, 0, 0, 0});
                 }
+                acc[c & 3] += (t[0] + t[1]) + (t[2] + t[3]);
             }
         }
 #pragma unroll
@@ -779,7 +794,7 @@ __device__ void bl_update_x(int n, int nrhs, int c0, int g, double *Xp, BlLds<MO
 #pragma unroll
     for (int c = 0; c < BL_MAXRHS; ++c) {
         const double v = bl_wave_max(xm[c]);
-        if (lane == 0) L.red[4 * BL_MAXRHS + wave * BL_MAXRHS + c] = v;
+        L.red[4 * BL_MAXRHS + wave * BL_MAXRHS + c] = v;
     }
     __syncthreads();
     if (tid < BL_MAXRHS)
@@ -855,10 +870,11 @@ void k_lu_ir_batched(int count, const int32_t *__restrict__ order, const int32_t
     for (;;) {
         if (threadIdx.x == 0) L.prob = (int)atomicAdd(&queue[0], 1u);
         __syncthreads();
-        // uniform: the problem's sizes and pointers stay in scalar registers and
-        // its loops are scalar branches.  As vector values they were the first
-        // to be spilled, and a spill at the end of a divergent branch was
-        // placed ahead of the restore of exec, which keeps lane 0's value only.
+        // Uniform, so that nothing derived from it is spilled early: a spill at
+        // the end of a divergent branch was placed ahead of the restore of
+        // exec, which keeps the branch's lanes only.  (With the body under an
+        // if instead of the continue below, every loop becomes a scalar branch
+        // and 4096 FP32 problems take 26.1 ms instead of 23.2.)
         const int pi = __builtin_amdgcn_readfirstlane(L.prob);
         __syncthreads();
         if (pi >= count) break;

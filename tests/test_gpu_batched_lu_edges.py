@@ -106,3 +106,22 @@ def test_nan_right_hand_side(tctx, torch_cuda, prec):
     assert be[0] > 1.0 and be[1] <= 1e-14
     assert st[0] == (0 if prec == la_hip.PREC_FP64 else la_hip.LA_NOT_CONVERGED) and st[1] == 0
     assert eta_of(a, y, b) <= 1e-14
+
+
+# The true residual of a converged refinement is the rounding of x and of the
+# residual's own sum.  Terms of variance s, roundings independent and of
+# variance at most u^2 / 3 of the partial sums: n / 4 sums of 4 (n / 4 * 10),
+# two levels of pairs (2 n), four chains of n / 64 sixteens (n^2 / 128), two
+# levels of pairs (2 n), and x (n).  Four chains of n / 4 terms would be
+# n^2 / 8 in place of n^2 / 128: 2.5 times as far off.
+def test_residual_rounding(tctx, torch_cuda):
+    n, g, count = 1024, 8, 4
+    bt = make_batch(torch_cuda, tctx, [n] * count, [g] * count, kappa=10, nrefl=64)
+    (x, st, it, be), = solve_batch(torch_cuda, tctx, bt, la_hip.PREC_FP32, tol=0.0, max_iter=4)
+    a, b = bt["A"].cpu().numpy(), bt["B"].cpu().numpy()
+    for i in range(count):
+        ai, bi = (v.astype(np.longdouble) for v in host_problem(bt, a, b, i))
+        xi = x[bt["offB"][i]:bt["offB"][i] + n * g].reshape(n, g).astype(np.longdouble)
+        s = ((ai ** 2) @ (xi ** 2)).mean() / n
+        var = (n / 4 * 10 + 4 * n + n * n / 128 + n) * s * 2.0 ** -106 / 3
+        assert ((bi - ai @ xi) ** 2).mean() <= var, i

@@ -1,8 +1,8 @@
 """Register spills of the batched LU kernels (batched_lu.hip, the only ones
-that spill more than a word).  The compiler can place a spill store at the
-head of the block that ends a divergent branch, before exec is restored: then
-only the branch's lanes are saved and the others reload stale values, which no
-diagnostic shows.  Checks the assembly of the kernels as built."""
+that spill more than a word).  The compiler can place a spill or a reload at
+the head of the block that ends a divergent branch, before exec is restored:
+then only the branch's lanes are saved or loaded and the others go on with
+stale values, which no diagnostic shows.  Checks the assembly of the kernels as built."""
 import os
 import re
 import shutil
@@ -15,7 +15,8 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 
 def misplaced(asm):
-    """Spill stores between a block's label and its restore of exec."""
+    """Spills and reloads between a block's label and its restore of exec (a
+    block that does vector work first is a branch's body, which ends there)."""
     found, kernel, head = [], None, None
     for line in asm.splitlines():
         m = re.match(r"(_Z\w+):", line)
@@ -27,16 +28,17 @@ def misplaced(asm):
             if re.match(r"\s+s_or_b64 exec, exec", line):
                 found += [(kernel, h) for h in head]
                 head = None
-            elif re.match(r"\s+s_(cbranch|branch|and_saveexec)", line):
-                head = None
-            elif re.match(r"\s+scratch_store.*Spill", line):
+            elif re.match(r"\s+scratch_(store.*Spill|load.*Reload)", line):
                 head.append(line.strip())
+            elif re.match(r"\s+(s_c?branch|v_|ds_|global_|scratch_|flat_)", line) and \
+                    not re.match(r"\s+v_(readlane|writelane|mov)_b", line):
+                head = None
     return found
 
 
 def test_finds_a_planted_one():
     good = "_Zk:\n.LBB0_1:\n\ts_or_b64 exec, exec, s[0:1]\n\tscratch_store_dword off, v1, off ; 4-byte Folded Spill\n"
-    bad = "_Zk:\n.LBB0_1:\n\tscratch_store_dword off, v1, off ; 4-byte Folded Spill\n\ts_or_b64 exec, exec, s[0:1]\n"
+    bad = "_Zk:\n.LBB0_1:\n\ts_mov_b32 s1, s2\n\tscratch_store_dword off, v1, off ; 4-byte Folded Spill\n\ts_or_b64 exec, exec, s[0:1]\n"
     assert misplaced(good) == [] and len(misplaced(bad)) == 1
 
 
