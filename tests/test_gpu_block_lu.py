@@ -69,3 +69,28 @@ def test_fp32_layout_edges(tctx, torch_cuda, n):
     # kappa * n * 2^-24 * growth << 1, so a second one reaches FP64 accuracy
     assert rep.status == la_hip.LA_OK and rep.iterations <= 3
     assert eta <= 1e-15 * n
+
+
+# Roundings per element: with pivots of 2^20, multipliers near 2^-20 and
+# elements that stay in [1, 2), each subtraction rounds an element by up to
+# half of 2^-52, independent of the others.  A column c of the block sees the
+# sums of four or more columns from the workgroups to its left and at most cw
+# single ones of its own; the quotient, the multiplier's own rounding and the
+# sums add less than four more.  (Column by column it would be c: 2.5 to 4
+# times the bound.)
+@pytest.mark.parametrize("m,cw", [(400, 32), (900, 16), (3000, 8), (5000, 4)])
+def test_roundings_per_element(tctx, torch_cuda, m, cw):
+    torch, n = torch_cuda, 256
+    rng = np.random.default_rng(m)
+    a = rng.uniform(1.25, 1.75, (m, n))
+    a[np.arange(n), np.arange(n)] = 2.0 ** 20
+    W = torch.from_numpy(a).cuda()
+    piv = torch.empty(m, dtype=torch.int64, device="cuda")
+    info = torch.zeros(4, dtype=torch.int32, device="cuda")
+    tctx.getrf_dev(W, piv, info)
+    assert info[1].item() == 0 and torch.equal(piv.cpu(), torch.arange(m))
+    lu = W.cpu().numpy().astype(np.longdouble)
+    l, u = np.tril(lu, -1)[n:], np.triu(lu[:n])
+    c = np.arange(192, 256)
+    r = a[n:, c] - l @ u[:, c]
+    assert ((r ** 2).mean(0) <= (c / 4 + cw + 4) * 2.0 ** -104 / 12 * 1.25).all()
