@@ -291,6 +291,8 @@ void k_getrf_panel(T *A, int64_t lda, int M, int NB, int R, int kglob, int64_t *
 
     stage_block(blk, LDB, A + (int64_t)rowbase * lda, lda, nrows, NB);
     if (tid == 0) s_abort = 0;
+    // a wait that is given up leaves no rows to move
+    if (w == 0 && tid == 0) swapmap[0] = 0;
     __syncthreads();
 
     // publish the candidate of step s (wave 0 only): rows >= s of column s
@@ -724,8 +726,8 @@ void k_apply_rowmoves(T *A, int64_t lda, int n, int c_lo, int c_hi,
         __syncthreads();                // the previous map's scatter is done
         if (tid == 0) s_cnt = (int)map[0];
         __syncthreads();
-        const int cnt = s_cnt;          // <= 2 * NB_IN <= blockDim.x
-        if (cnt == 0) continue;
+        const int cnt = min(s_cnt, 2 * NB_IN);
+        if (cnt <= 0) continue;
         for (int e = tid; e < cnt; e += blockDim.x) {
             s_dst[e] = map[1 + 2 * e];
             s_src[e] = map[2 + 2 * e];
@@ -776,7 +778,7 @@ void k_block_rowmoves(T *A, int64_t lda, int n, int c_lo, int c_hi, const int64_
     __shared__ int s_dst[BLK_MAP_MAX], s_src[BLK_MAP_MAX];
     const int tid = threadIdx.x;
     const int cnt = min((int)map[0], BLK_MAP_MAX);
-    if (cnt == 0) return;
+    if (cnt <= 0) return;
     for (int e = tid; e < cnt; e += 256) {
         s_dst[e] = (int)map[1 + 2 * e];
         s_src[e] = (int)map[2 + 2 * e];

@@ -141,6 +141,8 @@ void k_getrf_block(T *A, int64_t lda, int M, int nbo, int kglob, int64_t *ipiv, 
     }
     for (int i = tid; i < NB_OUT; i += NT) S.inv[i] = (uint16_t)i;
     if (tid == 0) { S.abort = 0; S.nmoves = 0; }
+    // a wait that is given up leaves no rows to move
+    if (g == 0 && tid == 0) swapmap[0] = 0;
 
     // swap of position k with the position of row rp (one thread); returns
     // that position

@@ -2,6 +2,7 @@
 // generators and the backward-error measurement.
 #include "la_common.hpp"
 #include <math.h>
+#include <stdlib.h>
 
 namespace lahip {
 
@@ -55,8 +56,11 @@ uint64_t spin_limit_ticks(la_ctx *ctx) {
     if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, ctx->device) !=
             hipSuccess || rate_khz <= 0)
         rate_khz = 100000;
-    // 5 s: far above any legitimate wait, short enough to fail fast.
-    return (uint64_t)rate_khz * 1000ull * 5ull;
+    // 5 s: far above any legitimate wait, short enough to fail fast.  (0 makes
+    // the waits of a launch give up at once, for tests of what follows.)
+    uint64_t ms = 5000;
+    if (const char *e = getenv("LAHIP_SPIN_LIMIT_MS")) ms = (uint64_t)std::max(0ll, atoll(e));
+    return (uint64_t)rate_khz * ms;
 }
 
 int fill_i32(la_ctx *ctx, int32_t *p, int64_t n, int32_t v) {
