@@ -1093,9 +1093,10 @@ constexpr size_t NOALLOC_PUB_OFF = NOALLOC_PANEL_BYTES + NOALLOC_MAX_K * sizeof(
 constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PUB_OFF + BLK_PUB_BYTES;
 
 // The block (M rows, nbo columns at Ablk) in one launch, then its L11^-1
-// blocks (linvs: null when no column right of the block needs them).  One workgroup per CU at most (the tall layouts fill a CU's
-// registers), nbo / cw of them, all resident at once on the whole device or
-// on the panel stream's CUs (checked by the caller).
+// blocks (linvs: null when no column right of the block needs them).  One
+// workgroup per CU at most (the tall layouts fill a CU's registers), nbo / cw
+// of them, all resident at once on the whole device or on the panel stream's
+// CUs (lookahead_from).
 template <typename T>
 static int launch_block(la_ctx *ctx, const BlockCfg &cfg, T *Ablk, int64_t lda, int M, int nbo,
                         int kglob, int64_t *d_ipiv, T *pub, uint64_t *pv, int64_t *map,
@@ -1226,7 +1227,6 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     const int64_t kmax = m < n ? m : n;
     // outer block from which the look-ahead schedule runs (kmax: never)
     const LookAhead *la = ext_ws ? nullptr : lookahead_streams(ctx);
-    int64_t K0la = kmax;
     // Which blocks go to the column-distributed kernel: by their rows alone,
     // so that every schedule and entry point factors a block the same way.
     // Not the factor of a matrix of at most NB_IN columns that one workgroup
@@ -1238,6 +1238,12 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     const int num_cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     auto block_for = [&](int64_t K0) -> const BlockCfg * {
         return pub ? block_cfg<T>(m - K0, num_cus) : nullptr;
+    };
+    // a kernel's workgroups that are not all resident wait for each other
+    // until the spin limit: what the panel stream cannot hold stays off it
+    auto fits_panel_stream = [&](int64_t K0) -> bool {
+        if (const BlockCfg *bc = block_for(K0)) return NB_OUT / bc->cw <= la->panel_cus;
+        return masked_panel_rpl<T>((int)(m - K0), la->panel_cus) > 0;
     };
     // panel workspace
     size_t slot_bytes = (size_t)2 * PANEL_MAXP * CAND_WORDS * sizeof(uint64_t);
@@ -1266,15 +1272,7 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
         else
             pub = (T *)ws_try(ctx, WS_PUB, BLK_PUB_BYTES);
     }
-    if (la)
-        for (int64_t K0 = 0; K0 + NB_OUT < kmax && K0 + NB_OUT < n; K0 += NB_OUT) {
-            const BlockCfg *bc = block_for(K0);
-            if (bc ? NB_OUT / bc->cw <= la->panel_cus
-                   : masked_panel_rpl<T>((int)(m - K0), la->panel_cus) > 0) {
-                K0la = K0;
-                break;
-            }
-        }
+    const int64_t K0la = la ? lookahead_from(kmax, n, fits_panel_stream) : kmax;
     PanelWS pw;
     char *b = (char *)base;
     pw.slots = (uint64_t *)b; b += al(slot_bytes);

@@ -469,23 +469,20 @@ void k_getrf_block(T *A, int64_t lda, int M, int nbo, int kglob, int64_t *ipiv, 
 // holds M rows is taken.  Rows x columns per workgroup fill 128 registers a
 // thread; past the tallest the row-distributed panels run (two columns per
 // workgroup would hand over on every second column).
-template <typename T, int NT, int RPT, int CW> static BlockCfg block_cfg_of()
+template <typename T, int I, int NT, int RPT> static BlockCfg block_cfg_of()
 {
-    return BlockCfg{NT * RPT, CW, (const void *)k_getrf_block<T, NT, RPT, CW>, NT,
-                    sizeof(BlockLds<T, NT, RPT, CW>)};
+    constexpr BlockShape s = sizeof(T) == 8 ? BLOCK_SHAPES_F64[I < 5 ? I : 0] : BLOCK_SHAPES_F32[I];
+    static_assert(s.rows == NT * RPT, "rows of the layout");
+    return BlockCfg{s.rows, s.cw, (const void *)k_getrf_block<T, NT, RPT, s.cw>, NT,
+                    sizeof(BlockLds<T, NT, RPT, s.cw>)};
 }
 template <typename T> const BlockCfg *block_cfg(int64_t M, int num_cus)
 {
     static const std::vector<BlockCfg> cfgs = [] {
-        std::vector<BlockCfg> v;
-        if constexpr (sizeof(T) == 8)
-            v = {block_cfg_of<T, 256, 2, 32>(), block_cfg_of<T, 256, 4, 16>(),
-                 block_cfg_of<T, 512, 4, 16>(), block_cfg_of<T, 512, 8, 8>(),
-                 block_cfg_of<T, 512, 16, 4>()};
-        else
-            v = {block_cfg_of<T, 256, 2, 32>(), block_cfg_of<T, 256, 4, 32>(),
-                 block_cfg_of<T, 512, 4, 32>(), block_cfg_of<T, 512, 8, 16>(),
-                 block_cfg_of<T, 512, 16, 8>(), block_cfg_of<T, 512, 32, 4>()};
+        std::vector<BlockCfg> v = {block_cfg_of<T, 0, 256, 2>(), block_cfg_of<T, 1, 256, 4>(),
+                                   block_cfg_of<T, 2, 512, 4>(), block_cfg_of<T, 3, 512, 8>(),
+                                   block_cfg_of<T, 4, 512, 16>()};
+        if constexpr (sizeof(T) == 4) v.push_back(block_cfg_of<T, 5, 512, 32>());
         for (auto &c : v)
             if (c.lds > allow_dynamic_lds(c.fn)) c.rows = 0;
         return v;

@@ -2,12 +2,11 @@
 // relaxed device-scope accesses of the exchanges between workgroups.
 #pragma once
 #include "la_common.hpp"
+#include "lu_schedule.hpp"
 
 namespace lahip {
 
 constexpr int PANEL_MAXP = 256;     // max cooperative workgroups in a panel
-constexpr int NB_IN = 64;           // inner panel width
-constexpr int NB_OUT = 256;         // outer block width (trailing GEMM K)
 
 // ---------------------------------------------------------------- keys
 // Ordered key for |v|: NaN -> 0 (never wins), otherwise bits(|v|)+1, so that
