@@ -1080,17 +1080,16 @@ constexpr size_t panel_ws_bytes(size_t elem)
 {
     return ws_align((size_t)2 * PANEL_MAXP * CAND_WORDS * sizeof(uint64_t)) + ws_align(256) +
            ws_align((size_t)2 * 2 * NB_IN * sizeof(uint64_t)) +
-           ws_align((size_t)(1 + 2 * BLK_MAP_MAX) * sizeof(int64_t)) +
-           ws_align((size_t)NB_OUT * sizeof(uint64_t)) +
+           ws_align((size_t)(1 + 4 * NB_IN) * sizeof(int64_t)) +
            ws_align((size_t)(NB_OUT / NB_IN) * NB_IN * NB_IN * elem);
 }
 
-// Fixed scratch of la_dgetrf_noalloc_dev: panel workspace, swap list,
-// published multipliers.
+// Fixed scratch of la_dgetrf_noalloc_dev: panel workspace, swap list, the
+// block kernel's slot.
 constexpr int64_t NOALLOC_MAX_K = 65536;
 constexpr size_t NOALLOC_PANEL_BYTES = panel_ws_bytes(sizeof(double));
 constexpr size_t NOALLOC_PUB_OFF = NOALLOC_PANEL_BYTES + NOALLOC_MAX_K * sizeof(int64_t);
-constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PUB_OFF + BLK_PUB_BYTES;
+constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PUB_OFF + BLK_SLOT_BYTES;
 
 // The block (M rows, nbo columns at Ablk) in one launch, then its L11^-1
 // blocks (linvs: null when no column right of the block needs them).  One
@@ -1225,13 +1224,13 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     if (m > INT32_MAX / 2 || n > INT32_MAX / 2)
         return set_error(ctx, LA_ERR_ARG, "getrf: extent too large");
     const int64_t kmax = m < n ? m : n;
-    // outer block from which the look-ahead schedule runs (kmax: never)
     const LookAhead *la = ext_ws ? nullptr : lookahead_streams(ctx);
     // Which blocks go to the column-distributed kernel: by their rows alone,
-    // so that every schedule and entry point factors a block the same way.
-    // Not the factor of a matrix of at most NB_IN columns that one workgroup
-    // holds (it keeps the reference's operation order), nor the factors with
-    // rounded update operands, whose in-block updates round as well.
+    // so that every schedule and entry point factors a block the same way
+    // (where the kernel's slot, pub, is there).  Not the factor of a matrix of
+    // at most NB_IN columns that one workgroup holds (it keeps the reference's
+    // operation order), nor the factors with rounded update operands, whose
+    // in-block updates round as well.
     const bool lp = upd_prec == LA_PREC_BF16 || upd_prec == LA_PREC_FP16;
     const bool exact = kmax <= NB_IN && (size_t)m * (kmax + 1) * sizeof(T) <= 96 * 1024;
     T *pub = nullptr;
@@ -1250,10 +1249,9 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     size_t row_bytes = 256;
     size_t diag_bytes = (size_t)2 * 2 * NB_IN * sizeof(uint64_t);
     size_t map_bytes = (size_t)(1 + 4 * NB_IN) * sizeof(int64_t);
-    size_t bmap_bytes = (size_t)(1 + 2 * BLK_MAP_MAX) * sizeof(int64_t);
     constexpr int RING = 2 * (NB_OUT / NB_IN);           // swap maps of two blocks
     auto al = [](size_t x) { return ws_align(x); };
-    static_assert(RING / 2 * ((1 + 4 * NB_IN) * 8) >= (1 + 2 * BLK_MAP_MAX) * 8,
+    static_assert(RING / 2 * ((1 + 4 * NB_IN) * 8) >= BLK_MAP_BYTES,
                   "a block's map fits the place of its panels' maps");
     void *base = ext_ws;
     int st;
@@ -1261,25 +1259,31 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     // update stream still applies block j (row moves, U12) while the panel
     // stream factors block j+1
     const size_t linv_bytes = al((size_t)(NB_OUT / NB_IN) * NB_IN * NB_IN * sizeof(T));
-    const size_t ring_bytes = la ? RING * al(map_bytes) + linv_bytes : 0;
+    // (under a workspace limit only where the row-distributed panels look
+    // ahead too, so that the limits that hold those hold this)
+    const int64_t K0rows = la ? lookahead_from(kmax, n, fits_panel_stream) : kmax;
+    const bool ring = la && (K0rows < kmax || (ctx->ws_limit == 0 && kmax > NB_OUT));
+    const size_t ring_bytes = ring ? RING * al(map_bytes) + linv_bytes : 0;
     if (!base && (st = ws_get(ctx, WS_PANEL, panel_ws_bytes(sizeof(T)) + ring_bytes, &base)))
         return st;
-    // the published multipliers; without room for them the row-distributed
-    // panels factor every block
+    // without room for the block kernel's slot the row-distributed panels
+    // factor every block
     if (!lp && !exact && block_cfg<T>(m - (kmax - 1) / NB_OUT * NB_OUT, num_cus)) {
         if (ext_ws)
             pub = (T *)((char *)ext_ws + NOALLOC_PUB_OFF);
         else
-            pub = (T *)ws_try(ctx, WS_PUB, BLK_PUB_BYTES);
+            pub = (T *)ws_try(ctx, WS_PUB, BLK_SLOT_BYTES);
     }
-    const int64_t K0la = la ? lookahead_from(kmax, n, fits_panel_stream) : kmax;
+    // outer block from which the look-ahead schedule runs (kmax: never)
+    const int64_t K0la = ring ? lookahead_from(kmax, n, fits_panel_stream) : kmax;
+    uint64_t *pv = (uint64_t *)((char *)pub + BLK_PUB_BYTES);
+    int64_t *bmap = (int64_t *)((char *)pv + BLK_PV_BYTES);
     PanelWS pw;
     char *b = (char *)base;
     pw.slots = (uint64_t *)b; b += al(slot_bytes);
     pw.rowbuf = b; b += al(row_bytes);
     pw.diagbuf = b; b += al(diag_bytes);
-    pw.swapmap = (int64_t *)b; b += al(bmap_bytes);
-    uint64_t *pv = (uint64_t *)b; b += al((size_t)NB_OUT * sizeof(uint64_t));
+    pw.swapmap = (int64_t *)b; b += al(map_bytes);
     T *linv_ring = (T *)b;
     b += linv_bytes;
     int64_t *swap_ring = (int64_t *)b;
@@ -1363,10 +1367,10 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
         const int64_t nbo = std::min<int64_t>(NB_OUT, kmax - K0);
         if (const BlockCfg *bc = block_for(K0)) {
             if ((st = launch_block<T>(ctx, *bc, A + K0 * lda + K0, lda, (int)(m - K0), (int)nbo,
-                                      (int)K0, d_ipiv, pub, pv, pw.swapmap, d_status, ticks,
+                                      (int)K0, d_ipiv, pub, pv, bmap, d_status, ticks,
                                       K0 + nbo < n ? linv_ring : (T *)nullptr)))
                 return st;
-            if ((st = launch_block_moves<T>(ctx, A, lda, n, K0, K0 + nbo, pw.swapmap, d_perm)))
+            if ((st = launch_block_moves<T>(ctx, A, lda, n, K0, K0 + nbo, bmap, d_perm)))
                 return st;
         } else if ((st = factor_block(K0, nbo, pw.swapmap, 0, linv_ring, 0, true))) {
             return st;

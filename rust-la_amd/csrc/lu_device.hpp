@@ -89,8 +89,13 @@ struct BlockCfg {
 };
 // The layout for a block of M rows whose workgroups find num_cus CUs, or null.
 template <typename T> const BlockCfg *block_cfg(int64_t M, int num_cus);
-// Published multipliers of a block: NB_OUT columns of the tallest layout.
+// What the block kernel needs beyond the row-distributed panels' workspace:
+// published multipliers (NB_OUT columns of the tallest layout), the words that
+// announce them, the swap map of a whole block.
 constexpr size_t BLK_PUB_BYTES = (size_t)NB_OUT * 8192 * sizeof(double);
+constexpr size_t BLK_PV_BYTES = NB_OUT * sizeof(uint64_t);
+constexpr size_t BLK_MAP_BYTES = (1 + 2 * BLK_MAP_MAX) * sizeof(int64_t);
+constexpr size_t BLK_SLOT_BYTES = BLK_PUB_BYTES + BLK_PV_BYTES + BLK_MAP_BYTES;
 
 // Inverses of the 64 x 64 diagonal triangles of a packed LU of order n (unit
 // lower, or upper), and X <- T^-1 X for a block of nbo <= NB_OUT rows with
