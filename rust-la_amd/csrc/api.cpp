@@ -22,6 +22,12 @@ int hip_fail(la_ctx *ctx, hipError_t e, const char *what) {
     return (e == hipErrorOutOfMemory) ? LA_ERR_NOMEM : LA_ERR_HIP;
 }
 
+bool capturing(la_ctx *ctx) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
+    return cap != hipStreamCaptureStatusNone;
+}
+
 int ws_get(la_ctx *ctx, int id, size_t bytes, void **out) {
     Workspace &w = ctx->ws[id];
     if (bytes == 0) bytes = 256;
@@ -30,7 +36,8 @@ int ws_get(la_ctx *ctx, int id, size_t bytes, void **out) {
         for (int i = 0; i < WS_COUNT; ++i)
             if (i != id) total += ctx->ws[i].size;
         Workspace &opt = ctx->ws[WS_PUB];
-        if (ctx->ws_limit > 0 && (int64_t)total > ctx->ws_limit && id != WS_PUB && opt.ptr) {
+        if (ctx->ws_limit > 0 && (int64_t)total > ctx->ws_limit && id != WS_PUB && opt.ptr &&
+            !opt.captured && !capturing(ctx)) {
             // the optional slot makes room
             hipError_t e = hipStreamSynchronize(ctx->stream);
             if (e != hipSuccess) return hip_fail(ctx, e, "ws_get sync");
@@ -61,11 +68,10 @@ int ws_get(la_ctx *ctx, int id, size_t bytes, void **out) {
 
 void *ws_try(la_ctx *ctx, int id, size_t bytes) {
     void *p = nullptr;
-    if (ctx->ws[id].size < bytes) {
+    if (capturing(ctx)) {
         // growing allocates and synchronises, which would end a capture
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
-        if (cap != hipStreamCaptureStatusNone) return nullptr;
+        if (ctx->ws[id].size < bytes) return nullptr;
+        ctx->ws[id].captured = true;
     }
     const std::string before = ctx->last_error;
     if (ws_get(ctx, id, bytes, &p) == LA_OK) return p;

@@ -47,6 +47,7 @@ constexpr uint64_t GOLDEN = 0x9E3779B97F4A7C15ULL;
 struct Workspace {
     void *ptr = nullptr;
     size_t size = 0;
+    bool captured = false;      // its address is in a captured graph (ws_try)
 };
 
 }  // namespace lahip
@@ -110,11 +111,16 @@ int hip_fail(la_ctx *ctx, hipError_t e, const char *what);
 int read_scratch(la_ctx *ctx, const int32_t *d, int32_t *h, int n);
 // LA_OK, or the sticky device error of a bounded wait (then cleared).
 int check_sticky(la_ctx *ctx);
+// Whether the context's stream is being captured into a graph.
+bool capturing(la_ctx *ctx);
 // Returns a device buffer of at least `bytes` from workspace slot `id`.
 int ws_get(la_ctx *ctx, int id, size_t bytes, void **out);
 // As ws_get, but for an optional buffer: null (and no error) when the
-// workspace limit or the device has no room for it.  WS_PUB is such a slot:
-// ws_get gives it back when another slot needs its room under the limit.
+// workspace limit or the device has no room for it, or when it would have to
+// grow inside a capture.  WS_PUB is such a slot: ws_get gives it back when
+// another slot needs its room under the limit, outside a capture and unless a
+// capture has used it (a replay of that graph writes to it as long as the
+// context lives).
 void *ws_try(la_ctx *ctx, int id, size_t bytes);
 
 #define LA_HIP_CHECK(ctx, expr)                                         \

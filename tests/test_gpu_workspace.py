@@ -1,5 +1,6 @@
-"""The dense solvers under a workspace limit: the paths taken where the optional
-buffers have no room, and what the limits hold.  Each test has a context of its own, whose workspaces start
+"""The dense solvers under a workspace limit and inside a capture: the
+paths taken where the optional buffers have no room, and what
+the limits hold.  Each test has a context of its own, whose workspaces start
 empty.  Results are compared with the unlimited context's (the same
 factorisation with other roundings) or with numpy."""
 import numpy as np
@@ -127,3 +128,67 @@ def test_qr_small_pool(fresh, torch_cuda, limit):
     want = np.linalg.lstsq(a, b, rcond=None)[0]
     # kappa(a) < 6: m n^(1/2) u kappa^2 and the reference's own error
     assert np.abs(X.cpu().numpy() - want).max() <= 700 * 18 * 2.0 ** -53 * 36
+
+
+# A captured factorisation and solve,
+# replayed on other data.  The context is warm, as captures need; `limit`:
+# between capture and replay another slot asks for room, which the captured
+# block slot must not give.
+@pytest.mark.parametrize("n", [200])
+@pytest.mark.parametrize("limit", [False, True])
+def test_captured_lu_solve(fresh, tctx, torch_cuda, n, limit):
+    torch = torch_cuda
+    A = torch.randn(n, n, dtype=torch.float64, device="cuda")
+    B = torch.randn(n, 4, dtype=torch.float64, device="cuda")
+    W, X = torch.empty_like(A), torch.empty_like(B)
+    piv = torch.empty(n, dtype=torch.int64, device="cuda")
+    info = torch.zeros(4, dtype=torch.int32, device="cuda")
+
+    def call():
+        W.copy_(A)
+        fresh.getrf_dev(W, piv, info)
+        fresh.getrs_dev(W, piv, B, X)
+
+    torch.cuda.synchronize()
+    with torch.cuda.stream(fresh.side):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=fresh.side):
+        call()
+    for k in range(3):
+        if limit:
+            _limit(fresh, 20 * MIB)
+            a = np.ones((700, 700))
+            with pytest.raises(la_hip.LaError) as e:
+                fresh.mul(a, a)                 # 11.8 MiB beside the 16 that stay
+            assert e.value.status == la_hip.LA_ERR_NOMEM
+        A.normal_()
+        B.normal_()
+        W0, p0 = _lu(tctx, torch, A)
+        X0 = torch.empty_like(B)
+        tctx.getrs_dev(W0, p0, B, X0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(W, W0) and torch.equal(piv, p0) and torch.equal(X, X0), k
+
+
+# A solve captured where the inverses' buffer would have to grow: the 64-row
+# exchange takes it.
+def test_captured_solve_without_room(fresh, torch_cuda):
+    torch, n = torch_cuda, 700
+    a = np.random.default_rng(2).standard_normal((n, n)) + 50 * np.eye(n)
+    W, piv = _lu(fresh, torch, torch.from_numpy(a).cuda())
+    B = torch.randn(n, 4, dtype=torch.float64, device="cuda")
+    X, b1, x1 = torch.empty_like(B), B[:, :1].contiguous(), torch.empty_like(B[:, :1])
+    torch.cuda.synchronize()
+    fresh.getrs_dev(W, piv, b1, x1)             # one column: the exchange's buffer
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=fresh.side):
+        fresh.getrs_dev(W, piv, B, X)
+    graph.replay()
+    torch.cuda.synchronize()
+    want = np.linalg.solve(a, B.cpu().numpy())
+    assert np.abs(X.cpu().numpy() - want).max() <= 1e-12 * np.abs(want).max()
