@@ -1156,6 +1156,9 @@ static const LookAhead *lookahead_streams(la_ctx *ctx)
     static LookAhead la[16];
     const char *off = getenv("LAHIP_LOOKAHEAD");
     if (off && atoi(off) == 0) return nullptr;
+    // a capture that forks to the masked streams ends in a crash inside the
+    // runtime's hipStreamEndCapture; the plain schedule's factor is the same
+    if (capturing(ctx)) return nullptr;
     if (ctx->device < 0 || ctx->device >= 16 || ctx->num_cus < 16 || ctx->num_cus % 8 != 0)
         return nullptr;
     std::lock_guard<std::mutex> g(mu);

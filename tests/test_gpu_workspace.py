@@ -130,11 +130,11 @@ def test_qr_small_pool(fresh, torch_cuda, limit):
     assert np.abs(X.cpu().numpy() - want).max() <= 700 * 18 * 2.0 ** -53 * 36
 
 
-# A captured factorisation and solve,
+# A captured factorisation and solve (the plain schedule, whatever its size),
 # replayed on other data.  The context is warm, as captures need; `limit`:
 # between capture and replay another slot asks for room, which the captured
 # block slot must not give.
-@pytest.mark.parametrize("n", [200])
+@pytest.mark.parametrize("n", [200, 700])
 @pytest.mark.parametrize("limit", [False, True])
 def test_captured_lu_solve(fresh, tctx, torch_cuda, n, limit):
     torch = torch_cuda
