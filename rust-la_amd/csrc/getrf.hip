@@ -1094,8 +1094,8 @@ constexpr size_t NOALLOC_SCRATCH_BYTES = NOALLOC_PUB_OFF + BLK_SLOT_BYTES;
 // The block (M rows, nbo columns at Ablk) in one launch, then its L11^-1
 // blocks (linvs: null when no column right of the block needs them).  One
 // workgroup per CU at most (the tall layouts fill a CU's registers), nbo / cw
-// of them, all resident at once on the whole device or on the panel stream's
-// CUs (lookahead_from).
+// of them, all resident at once on the CUs of the caller's stream (home_cus)
+// or on the panel stream's (lookahead_from).
 template <typename T>
 static int launch_block(la_ctx *ctx, const BlockCfg &cfg, T *Ablk, int64_t lda, int M, int nbo,
                         int kglob, int64_t *d_ipiv, T *pub, uint64_t *pv, int64_t *map,
@@ -1279,6 +1279,8 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     }
     // outer block from which the look-ahead schedule runs (kmax: never)
     const int64_t K0la = ring ? lookahead_from(kmax, n, fits_panel_stream) : kmax;
+    // CUs of the caller's stream, for the blocks of the plain schedule
+    const int home_cus = pub && K0la > 0 ? stream_cus(ctx) : num_cus;
     uint64_t *pv = (uint64_t *)((char *)pub + BLK_PUB_BYTES);
     int64_t *bmap = (int64_t *)((char *)pv + BLK_PV_BYTES);
     PanelWS pw;
@@ -1368,7 +1370,8 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     // plain schedule
     for (int64_t K0 = 0; K0 < K0la; K0 += NB_OUT) {
         const int64_t nbo = std::min<int64_t>(NB_OUT, kmax - K0);
-        if (const BlockCfg *bc = block_for(K0)) {
+        const BlockCfg *bc = block_for(K0);
+        if (bc && NB_OUT / bc->cw <= home_cus) {
             if ((st = launch_block<T>(ctx, *bc, A + K0 * lda + K0, lda, (int)(m - K0), (int)nbo,
                                       (int)K0, d_ipiv, pub, pv, bmap, d_status, ticks,
                                       K0 + nbo < n ? linv_ring : (T *)nullptr)))

@@ -146,6 +146,8 @@ struct ProfScope {
 // on gfx950); returns that limit in bytes and leaves no sticky HIP error.
 size_t allow_dynamic_lds(const void *kernel);
 uint64_t spin_limit_ticks(la_ctx *ctx);
+// CUs that the context's stream may use (its CU mask, or all).
+int stream_cus(la_ctx *ctx);
 int fill_i32(la_ctx *ctx, int32_t *p, int64_t n, int32_t v);
 int fill_u64(la_ctx *ctx, uint64_t *p, int64_t n, uint64_t v);
 int iota_u64(la_ctx *ctx, uint64_t *p, int64_t n);

@@ -63,6 +63,18 @@ uint64_t spin_limit_ticks(la_ctx *ctx) {
     return (uint64_t)rate_khz * ms;
 }
 
+int stream_cus(la_ctx *ctx) {
+    const int all = ctx->num_cus > 0 ? ctx->num_cus : 256;
+    uint32_t mask[32] = {};
+    if (hipExtStreamGetCUMask(ctx->stream, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return all;
+    }
+    int n = 0;
+    for (int i = 0; i < std::min(all, 32 * 32); ++i) n += (mask[i / 32] >> (i % 32)) & 1;
+    return n > 0 ? n : all;
+}
+
 int fill_i32(la_ctx *ctx, int32_t *p, int64_t n, int32_t v) {
     if (n <= 0) return LA_OK;
     hipLaunchKernelGGL(k_util_fill_i32, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, p, n, v);

@@ -1,8 +1,10 @@
-"""The dense solvers under a workspace limit and inside a capture: the
-paths taken where the optional buffers have no room, and what
+"""The dense solvers under a workspace limit, inside a capture and on a stream
+of few CUs: the paths taken where the optional buffers have no room, and what
 the limits hold.  Each test has a context of its own, whose workspaces start
 empty.  Results are compared with the unlimited context's (the same
 factorisation with other roundings) or with numpy."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -192,3 +194,21 @@ def test_captured_solve_without_room(fresh, torch_cuda):
     torch.cuda.synchronize()
     want = np.linalg.solve(a, B.cpu().numpy())
     assert np.abs(X.cpu().numpy() - want).max() <= 1e-12 * np.abs(want).max()
+
+
+# A caller's stream with one CU of each XCD: a block of 16 workgroups goes to
+# the row-distributed panel (8 of 128 rows), one of 8 stays.
+@pytest.mark.parametrize("shape", [(900, 200), (500, 200)])
+def test_stream_of_few_cus(tctx, torch_cuda, shape):
+    torch = torch_cuda
+    hip = tctx.lib                              # its HIP runtime's symbols with it
+    s, words = ctypes.c_void_p(), (ctypes.c_uint32 * 8)(0xff)
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(s), 8, words) == 0
+    c = la_hip.Context(0)
+    c.set_stream(s.value)
+    A = torch.randn(shape, dtype=torch.float64, device="cuda")
+    W0, p0 = _lu(tctx, torch, A)
+    W1, p1 = _lu(c, torch, A)
+    assert torch.equal(p0, p1) and _backward_stable(torch, A, W1, p1)
+    c.close()
+    assert hip.hipStreamDestroy(s) == 0
