@@ -99,11 +99,11 @@ constexpr size_t BLK_SLOT_BYTES = BLK_PUB_BYTES + BLK_PV_BYTES + BLK_MAP_BYTES;
 
 // Inverses of the 64 x 64 diagonal triangles of a packed LU of order n (unit
 // lower, or upper), and X <- T^-1 X for a block of nbo <= NB_OUT rows with
-// them (trsm_block.hip).
+// them (trsm_block.hip); refine: with one correction per 64 rows.
 template <typename T>
 int launch_block_inv(la_ctx *ctx, bool upper, const T *Tm, int64_t ldt, int64_t n, T *inv);
 template <typename T>
 int launch_trsm_block(la_ctx *ctx, bool upper, const T *Tm, int64_t ldt, const T *inv, int nbo,
-                      T *B, int64_t ldb, int64_t ncols);
+                      T *B, int64_t ldb, int64_t ncols, bool refine = false);
 
 }  // namespace lahip

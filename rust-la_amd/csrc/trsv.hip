@@ -419,10 +419,13 @@ int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ld
     double *inv = (double *)base;
     if ((st = launch_block_inv<double>(ctx, !lower, Tm, ldt, n, inv))) return st;
     const int64_t nblk = ceil_div(n, NB_OUT);
+    // one correction per 64 rows up to the order where the residual falls
+    // below k_trsv's without it (n = 700: 1.0 to 1.1 times, 1500: 0.3 to 0.6)
+    const bool refine = n <= 1024;
     for (int64_t s = 0; s < nblk; ++s) {
         const int64_t R0 = (lower ? s : nblk - 1 - s) * NB_OUT, R1 = std::min<int64_t>(n, R0 + NB_OUT);
         if ((st = launch_trsm_block<double>(ctx, !lower, Tm + R0 * (ldt + 1), ldt, inv + R0 * TB,
-                                            (int)(R1 - R0), X + R0 * ldx, ldx, nrhs)))
+                                            (int)(R1 - R0), X + R0 * ldx, ldx, nrhs, refine)))
             return st;
         const int64_t r0 = lower ? R1 : 0, rows = lower ? n - R1 : R0;
         if ((st = gemm_rm<double>(ctx, rows, nrhs, R1 - R0, -1.0, Tm + r0 * ldt + R0, ldt,

@@ -34,3 +34,24 @@ def test_integer_triangles(ctx, n):
     lu = np.tril(low, -1) + up
     x = ctx.lu_solve(lu, np.arange(n, dtype=np.uint64), low @ (up @ xs))
     assert np.array_equal(x, xs)
+
+
+# Upper triangles of factors with singular values in [1e-6, 1] (L the identity):
+# after the correction x carries its own rounding (at most u, rms u / 3^(1/2))
+# and that of the residual, a sum of at most 100 terms whose rounding is below
+# a tenth of u of the sum of their magnitudes: 0.58 + 0.07 u.
+@pytest.mark.parametrize("n", [65, 100])
+def test_small_solve_residual(tctx, torch_cuda, n):
+    torch = torch_cuda
+    rng = np.random.default_rng(n)
+    total = []
+    for k in range(12):
+        q1, q2 = (np.linalg.qr(rng.standard_normal((n, n)))[0] for _ in range(2))
+        lu = torch.linalg.lu_factor(torch.from_numpy((q1 * 1e-6 ** np.linspace(0, 1, n)) @ q2))[0]
+        W, B = torch.triu(lu).cuda(), torch.randn(n, 16, dtype=torch.float64, device="cuda")
+        X, piv = torch.empty_like(B), torch.arange(n, device="cuda")
+        tctx.getrs_dev(W, piv, B, X)
+        torch.cuda.synchronize()
+        u, x, b = (t.cpu().numpy().astype(np.longdouble) for t in (W, X, B))
+        total.append(((b - u @ x) / (np.abs(u) @ np.abs(x))) ** 2)
+    assert np.mean(total) ** 0.5 <= 0.65 * 2.0 ** -53
