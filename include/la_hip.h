@@ -64,7 +64,14 @@ int         la_ctx_set_stream(la_ctx *ctx, void *hip_stream);
 const char *la_status_string(int status);
 const char *la_ctx_last_error(la_ctx *ctx);
 int         la_device_info(la_ctx *ctx, int *num_cus, int64_t *hbm_bytes, int *clock_khz);
-/* Cap (bytes) on the context's grow-only device workspace; 0 = no cap. */
+/* Cap (bytes) on the context's grow-only device workspace; 0 = no cap.  Two
+ * buffers are optional and left out under a cap that has no room for them:
+ * the 16 MiB in which the LU's block kernel exchanges columns (without it, or
+ * inside a capture before any call has allocated it, every block is factored
+ * by the row-distributed panels), and the inverses of the triangular solves by
+ * 256-row blocks (any cap that they would have to grow under).  The results
+ * are then rounded differently: last bits, and the pivot where two candidates
+ * are equal to within rounding. */
 int         la_ctx_set_workspace_limit(la_ctx *ctx, int64_t bytes);
 
 /* ------------------------------------------------ kernel timing harness
@@ -203,12 +210,20 @@ int la_dgemm_dev(la_ctx *ctx, int64_t m, int64_t n, int64_t k,
  * factored by at most min(256, CUs) co-resident workgroups of at most 192
  * rows each (FP64; 256 for the FP32 factor of la_dgesv_ir_dev), so
  * m <= 49152 on a 256-CU MI355X (65536 for the FP32 factor); beyond it the
- * call returns LA_ERR_ARG before launching anything.  Outer blocks whose rows
- * fit 96 CUs run with look-ahead on two process-wide streams with
- * complementary CU masks (panels of block j+1 beside the update of block j),
- * ordered after earlier work on ctx's stream and before later work on it by
- * events, so the call stays stream-ordered; the factor is bit-identical to
- * the single-stream schedule's, which LAHIP_LOOKAHEAD=0 selects. */
+ * call returns LA_ERR_ARG before launching anything.  From the first outer
+ * block that fits 96 CUs with every later one, blocks run with look-ahead on
+ * two process-wide streams with complementary CU masks (block j+1 factored
+ * beside the update of block j), ordered after earlier work on ctx's stream
+ * and before later work on it by events, so the call stays stream-ordered; the
+ * factor is bit-identical to the single-stream schedule's, which
+ * LAHIP_LOOKAHEAD=0 selects and a capture of ctx's stream always gets.  On a
+ * stream with a CU mask a block that needs more workgroups (up to 64) than the
+ * mask has CUs is factored by the row-distributed panels, rounded differently
+ * as under a workspace cap.  The workgroups of a block or panel wait for each
+ * other and are all resident at once only if other work (of another stream or
+ * process) leaves them CUs; a wait that lasts longer than 5 s
+ * (LAHIP_SPIN_LIMIT_MS) is given up with status LA_ERR_TIMEOUT and A
+ * undefined. */
 int la_dgetrf_dev(la_ctx *ctx, int64_t m, int64_t n, double *A, int64_t lda,
                   uint64_t *d_piv, int32_t *d_info);
 
@@ -216,8 +231,9 @@ int la_dgetrf_dev(la_ctx *ctx, int64_t m, int64_t n, double *A, int64_t lda,
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * factorisation, its kernels and its results are those of la_dgetrf_dev;
- * its workspace (panel exchange slots, swap map, L11^-1 blocks, swap list)
- * is a fixed per-device scratch array of about 1.2 MiB instead of the
+ * its workspace (panel exchange slots, swap map, L11^-1 blocks, swap list,
+ * the block kernel's exchange) is a fixed per-device scratch array of about
+ * 17 MiB instead of the
  * context's grow-only workspace.  Limit: min(m, n) <= 65536 (LA_ERR_ARG
  * beyond).  The scratch is shared by every call on one device and keeps the
  * last call's contents (each call resets what it reads first): calls that
@@ -229,7 +245,9 @@ int la_dgetrf_noalloc_dev(la_ctx *ctx, int64_t m, int64_t n, double *A, int64_t 
 
 /* Solve with a device-resident packed LU; X (m x nx, ld ldx) must not
  * alias B.  If d_status is non-NULL it receives LA_SINGULAR when U has an
- * exact zero on its diagonal (the reference's None, lu.rs:241-243). */
+ * exact zero on its diagonal (the reference's None, lu.rs:241-243).  A column's
+ * last bits may depend on nx: one column above n = 512 is solved 64 rows at a
+ * time, several columns (and one up to n = 512) 256 rows at a time. */
 int la_dgetrs_dev(la_ctx *ctx, int64_t m, int64_t n, const double *LU, int64_t ldlu,
                   const uint64_t *d_piv, int64_t nx, const double *B, int64_t ldb,
                   double *X, int64_t ldx, int32_t *d_status);

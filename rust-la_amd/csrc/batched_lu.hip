@@ -27,7 +27,7 @@
 // on ties) in the working precision.
 //
 // What bounds it: 4096 problems, n log-uniform in [32, 1024], 1-8 right-hand
-// sides, take 23.1 ms in FP32 (FP64 28.5, FP16 39.3; 57, 61.5 and 136 before
+// sides, take 23.2 ms in FP32 (FP64 28.9, FP16 36.8; 57, 61.5 and 136 before
 // the products with few columns went to MFMA, panels to blocks of eight
 // columns and updates to outer blocks of 64).  Of the FP32 time the updates
 // are 6.4 ms, panels 4.5, substitution 3.4 and residuals 3.0 (each reads its
@@ -307,7 +307,7 @@ __device__ void bl_getrf(int n, typename BlCfg<MODE>::T *__restrict__ W, int *__
                 if (pos[s] == ppos) pos[s] = j;
                 else if (pos[s] == j) pos[s] = ppos;
             }
-            if (!(piv != (T)0)) {           // exact zero (or NaN) pivot: no scaling
+            if (!(piv != (T)0)) {           // exact zero pivot: no scaling (a NaN scales)
                 if (tid == 0) L.singular = 1;
                 return;
             }

@@ -4,21 +4,25 @@
 // the pivot of column j is the FIRST row at or below j with the strictly
 // largest |a_ij| (ties go to the lowest row index); a NaN never displaces the
 // current candidate, so a NaN on the diagonal stays the pivot; rows are
-// swapped whole; the multipliers are a_ij / a_jj (a true division) and are
+// swapped whole; the multipliers are a_ij / a_jj (by division where one
+// workgroup holds the matrix, elsewhere from the pivot's reciprocal) and are
 // left unscaled when the pivot is exactly zero.
 //
-// Structure (two-level blocking):
+// Structure:
 //   for each outer block of NB_OUT columns
+//     block kernel       : the whole block in one launch, columns distributed
+//                          over workgroups (getrf_block.hip); where it does
+//                          not hold the rows, or its slot has no room:
 //     for each inner panel of NB_IN columns inside it
-//       panel kernel     : cooperative, P workgroups, rows held in LDS,
-//                          one cross-workgroup exchange per column
+//       panel kernel     : P co-resident workgroups, rows held in LDS, one
+//                          cross-workgroup exchange per column
 //       row-swap kernel  : net permutation of the panel applied to every
 //                          column outside the panel and to the perm vector
 //       trsm + gemm      : update the rest of the outer block
 //     u12 + gemm         : U12 = L11^-1 A12 (one kernel per block),
 //                          A22 -= L21 U12 (MFMA, K = NB_OUT)
-// Once the remaining rows fit the CUs reserved for panels (the panel
-// stream's), outer blocks overlap: block j+1's panels run on those CUs while
+// Once this and every later block fit the CUs reserved for panels (the panel
+// stream's), outer blocks overlap: block j+1 is factored on those CUs while
 // the other CUs apply block j (look-ahead; see getrf_core).
 #include "lu_device.hpp"
 #include <mutex>
@@ -153,7 +157,7 @@ __device__ void invert_unit_lower_wave(const T *L, int ldl, int nb, T *out)
 
 // ------------------------------------------------------------- panel kernel
 // Factors the M x NB panel whose top-left element is A (row-major, lda),
-// global column/row offset kglob, with P cooperative workgroups; workgroup
+// global column/row offset kglob, with P co-resident workgroups; workgroup
 // w owns panel rows [w*R, min(w*R+R, M)) in LDS for the whole kernel and
 // its first wavefront owns the per-column critical path (R <= 64*RPL).
 //
@@ -182,7 +186,7 @@ __device__ void invert_unit_lower_wave(const T *L, int ldl, int nb, T *out)
 // step kglob = 0 mod 4, whose first two steps (bit 1 clear) reject it.
 //
 // Per column, once the winner p is known: rows j and p are swapped, then the
-// first wavefront forms the multipliers (true division, skipped for a zero
+// first wavefront forms the multipliers (one reciprocal; skipped for a zero
 // pivot), updates column j+1, picks the next local candidate, brings that
 // row (and row j+1 if owned) fully up to date and publishes step j+1 before
 // the whole workgroup applies the rest of the rank-1 update, so the bulk of
@@ -900,7 +904,7 @@ struct PanelWS {
     void *rowbuf;
     void *diagbuf;
     int64_t *swapmap;
-    int last_p = 1 << 30;       // workgroups of the previous cooperative panel
+    int last_p = 1 << 30;       // workgroups of the previous row-distributed panel
 };
 
 
@@ -1142,8 +1146,9 @@ static int launch_block_moves(la_ctx *ctx, T *A, int64_t lda, int64_t n, int64_t
 // pair serves every factorisation: 12 CUs per XCD (the default) is what the
 // row-distributed panels need (FP64 n = 16384: 99 ms, 114 with 8), and a second
 // pair of 8 for the factorisations whose blocks need only 64 CUs (FP32-IR
-// n = 16384: 71.1 against 73.6 ms) slows whichever pair a process uses second
-// by a tenth (BF16 + GMRES n = 16384 115 -> 126 ms, FP32-IR 62 -> 69 ms).
+// n = 16384: 71.1 against 73.6 ms, before the block kernel summed the left
+// columns' products: 76.7 now) slows whichever pair a process uses second by a
+// tenth (BF16 + GMRES n = 16384 115 -> 126 ms, FP32-IR 62 -> 69 ms).
 struct LookAhead {
     hipStream_t panel = nullptr, update = nullptr;
     int panel_cus = 0;
@@ -1205,10 +1210,11 @@ struct StreamSwap {
 // bytes, or null for the context's grow-only workspace.
 //
 // Outer blocks run one of two schedules.  The plain schedule factors a block
-// and then updates everything to its right, all on ctx->stream.  Once the
-// remaining rows fit the panel stream's CUs, blocks run with look-ahead: the
-// panel stream factors block j+1 (panels, their row moves inside the block,
-// the in-block updates) while the update stream applies block j to the
+// and then updates everything to its right, all on ctx->stream.  From the
+// first outer block that fits the panel stream's CUs with every later one
+// (lookahead_from), blocks run with look-ahead: the panel stream factors block
+// j+1 (the block kernel, or panels, their row moves inside the block and the
+// in-block updates) while the update stream applies block j to the
 // columns right of block j+1.  Per block j the update stream does, in order:
 // block j's row moves, U12 = L11^-1 A12 and update on block j+1's columns
 // (after which block j+1 may start), then block j's row moves on the columns
@@ -1403,10 +1409,13 @@ int getrf_core(la_ctx *ctx, int64_t m, int64_t n, T *A, int64_t lda, int64_t *d_
     // large the panel stream finishes block j+1 long before the update
     // stream finishes block j's update, so it takes the rightmost columns of
     // that update once block j+1 is factored.  The share is sized from a
-    // rate model (GEMM FLOP/s per CU at K = 256 and panel time per column,
-    // both measured on MI355X at n = 16384) so that both streams finish
-    // together (scaling the modelled share by 0.5 or 1.5 was slower); it never includes the columns of
-    // blocks j+1 and j+2, which the update stream needs first.  Fencing: the
+    // rate model (GEMM FLOP/s per CU at K = 256, and the time per column of
+    // the row-distributed panels, both measured on MI355X at n = 16384; the
+    // block kernel's columns are faster, 2.2-4.0 us, and the share it leaves
+    // smaller than it could be) so that both streams finish together (with
+    // those panels, scaling the modelled share by 0.5 or 1.5 was slower); it
+    // never includes the columns of blocks j+1 and j+2, which the update
+    // stream needs first.  Fencing: the
     // panel stream's share waits for block j's U12 there (ev_u12); the update
     // stream waits for the share (ev_share) before block j+1's row moves,
     // which rewrite rows of block j's L21 that the share reads.

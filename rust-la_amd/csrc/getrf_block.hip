@@ -40,7 +40,7 @@ namespace lahip {
 // first and then taken from the element: one after the other they rounded
 // every element up to 255 times, and the error of an FP32 factor of n = 16384
 // with singular values in [1e-6, 1] was 1.6 times that of 64-column panels with
-// GEMM updates between them (now 0.6 times; the batches cost 2-8% of a
+// GEMM updates between them (now 0.6 times; the batches cost 2-9% of a
 // factorisation).  The batch is fixed, not what happens to be published, so
 // that a factor does not depend on timing.  Its pivot rows, as they stand
 // before it, are brought up to date by a triangular solve of order LB.
@@ -58,8 +58,9 @@ namespace lahip {
 // the reciprocal and the LDS reads of the pivot row; per CW columns the
 // hand-over to the next workgroup (a store's way to memory, the poll, the
 // load of the multipliers).  Measured on the panel stream, 256 columns:
-// FP64 780 us at 4096-8192 rows, 540 at 2048-4096, 570 at 1024-2048, 400 at
-// 256-512; FP32 890 at 8192-16384, 630 at 4096-8192.  Four row-distributed
+// FP64 920 us at 4096-8192 rows (767 with the left columns applied one at a
+// time), 560 at 2048-4096, 590 at 1024-2048, 480 below; FP32 1040 at 8192-16384
+// (888), 645 at 1024-8192, 500 at 512-1024, 390 below.  Four row-distributed
 // panels with their in-block row moves, TRSM and GEMM took 1.1-1.5 ms.
 //
 // Layout: NT x RPT rows and CW columns so that a thread's RPT x CW elements

@@ -209,9 +209,10 @@ int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ld
 // right-hand-side counts from which the LU solves use trsm_blocked
 constexpr int64_t TRSM_MIN_RHS = 2, TRSM_MIN_N = 65;
 // and the order up to which they use it for one right-hand side too: k_trsv
-// starts with the inversion of a diagonal block (40 us) and goes on at 4 us
-// per 64 rows, trsm_blocked takes 6 us and 27 per 256 rows (n = 256: 54
-// against 23 us a triangle, equal near n = 700)
+// starts with the inversion of a diagonal block (40 us a triangle) and goes on
+// at 2-4 us per 64 rows, trsm_blocked takes 7 us and, with its correction,
+// 27 per 256 rows (both triangles, us: n = 65 96 against 35, 256 112 against
+// 65, 512 137 against 132)
 constexpr int64_t TRSM_ONE_RHS_MAX_N = 512;
 static inline bool trsm_wins(int64_t n, int64_t nrhs)
 {

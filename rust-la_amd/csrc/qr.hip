@@ -675,7 +675,7 @@ int qr_ws(la_ctx *ctx, int64_t m, int64_t n, int64_t wcols, QrWs &w)
     const size_t fixed = bv + QR_G_BYTES + bw + bp + bd + bs + bsl;
     // room for every partial; under a workspace limit the least that holds a
     // panel's Gram partials beside one chunk of products (fewer, longer
-    // chunks: qr_chunks)
+    // chunks: what fits decides their number where the update is launched)
     const size_t full = (size_t)QRP_MAXP * QR_G_BYTES + (size_t)VT_MAXCHUNK * bw;
     const size_t least = std::max((size_t)VT_MAXCHUNK * bw, (size_t)QRP_MAXP * QR_G_BYTES) + bw +
                          2 * QR_G_BYTES;

@@ -132,7 +132,8 @@ void k_block_inv(const T *Tm, int64_t ldt, int64_t nbo, T *inv)
 // every sixteen) one 64 x 64 stage ahead, and none depends on X.
 // Bound by the chain of ten stages and their latency: as U12 it precedes the
 // next block's update on the LU's critical path.  256 columns take 16 us in
-// FP64 (47 with the products on FMAs from LDS) and 13 in FP32 (36).
+// FP64 (47 with the products on FMAs from LDS; 26 with REFINE) and 13 in FP32
+// (36).
 // REFINE: X_b is corrected once, X_b += inv(T_bb) (Y - T_bb X_b).  The residual
 // of a solve with the inverses as they are is 1.0 to 1.3 times that with
 // inverses by substitution for random matrices of n <= 512 (2.4 times for

@@ -397,9 +397,9 @@ int trsv_blocked(la_ctx *ctx, char uplo, bool trans, bool unit, int64_t n, const
 // once per 64 rows and is bound by that exchange, which grows with the
 // right-hand sides: both triangles of n = 8192 with 16 take it 7.0 ms, of
 // n = 1500 with 7 0.84 ms, against 2.8 and 0.4 here.  With one right-hand side
-// k_trsv wins above n = 512 (trsm_wins); it also serves up to NR when a workspace limit is
-// set, under which the inverses could take the room of a later call, and when
-// they would have to be allocated inside a capture.
+// k_trsv wins above n = 512 (trsm_wins); it also serves up to NR when a
+// workspace limit is set, under which the inverses could take the room of a
+// later call, and when they would have to be allocated inside a capture.
 int trsm_blocked(la_ctx *ctx, char uplo, int64_t n, const double *Tm, int64_t ldt, int64_t nrhs,
                  double *X, int64_t ldx)
 {
